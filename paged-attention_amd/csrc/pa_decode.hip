@@ -56,8 +56,8 @@
 //   * Split rows are merged by the split kernel itself when the plan allows
 //     (block_merge 1 and 2): a unit's split segments are only its first and
 //     last, so each wave keeps at most two partials (and their LSEs) in LDS;
-//     after one barrier every thread of the block merges one head-dim element
-//     of each split row. A row inside the block (e.g. 32 rows x 8 kv heads x
+//     after one barrier the waves merge the block's split rows side by side
+//     (tasks of 256 elements of one row). A row inside the block (e.g. 32 rows x 8 kv heads x
 //     8192 tokens over 2048 units) is then complete; a row that spans blocks
 //     (up to 8) leaves one device-coherent partial per block, and the last
 //     of its blocks to arrive (a per-row counter) combines them, in block
@@ -308,19 +308,159 @@ __device__ __forceinline__ void store_coherent(float* p, float v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Block-level merge after the split loop. slot_item holds, per wave, the
-// (row, kv head) item of its first (slot 0) and last (slot 1) segment when that
-// segment is a split one, else -1 (slot_seg: that segment's index); part / lse
-// hold the slot's normalized partial rows and base-2 LSEs, written to LDS by
-// the wave that computed them. Each thread owns one head-dim element (two for
-// G = 8) of every item and reads that element of all 16 slots at once, with
-// the LSEs and slot items (one LDS round trip). An item's weights
-// 2^(lse - max) depend only on the slot and the head, and a wave's 64
-// elements share one head, so lane j of each wave computes slot j's weight
-// once (0 outside the item) and the element sums take them as wave-uniform
-// operands: the base-2 LSE-weighted average of the item's partials in this
-// block (decode_kernels.cuh:409-432), summed in slot order. No branch depends
-// on a slot.
+// Device-coherent 16-byte store (the same cache policy as store_coherent's
+// atomic stores, four values at a time).
+__device__ __forceinline__ void store_coherent16(const __amdgpu_buffer_rsrc_t rs, int byte_off, const f32x4 v) {
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rs, byte_off, 0, kAuxCoherent);
+}
+
+// One split segment that a wave left in LDS: its (row, kv head) item (-1: the
+// slot is empty), its index in the plan, and the item's first segment and
+// segment count. Read as one 16-byte vector.
+struct alignas(16) Slot {
+    int item, seg, s0, n;
+};
+
+// An item of this block that spans blocks.
+struct Span {
+    int item, s0, n, u0;   // u0: the unit of its first segment
+};
+
+// The last block of a spanning item combines the item's block partials (block
+// j's sits at the item's first segment in block j). They are summed in NGR
+// states per 16-byte dim vector, state g taking every NGR-th block from g on,
+// each with one coherent 16-byte load of the row and one of its LSE, all issued
+// before the first is used (one round trip), with a running maximum in block
+// order; the states of a vector then meet in a fixed tree (1, 2, 4, 8 apart).
+// A block that is last for one item has one state per thread; a block that is
+// last for two has S = 2 states per thread and half its threads on each item,
+// side by side. The tree's sums are rounded the same from both sides
+// (no contraction), so the result depends neither on S nor on timing.
+template <int G, int S>
+__device__ __forceinline__ void combine_blocks(const pa_decode_params& p, const Span& it, int t) {
+#pragma clang fp contract(off)
+    constexpr int NO  = G * kHeadDim;
+    constexpr int NV  = NO / 4;                   // 16-byte vectors of one block partial
+    constexpr int NGR = 64 * kWaves / NV;         // states of one vector (16, 8, 4, 2 for G = 1, 2, 4, 8)
+    constexpr int LPV = NGR / S;                  // lanes sharing one vector
+    constexpr int U   = NGR >= 8 ? 1 : 8 / NGR;   // loads per state and round (8 blocks)
+    static_assert(S == 1 || S == 2, "one or two states per thread");
+    static_assert(LPV >= 1 && LPV <= 16 && (LPV & (LPV - 1)) == 0, "the lanes of a vector lie in one DPP row");
+    const int li = t % LPV;
+    const int vi = t / LPV;
+    const int hh = 4 * vi / kHeadDim;            // query head of the vector
+    const int j0 = it.u0 / kWaves, j1 = (it.u0 + it.n - 1) / kWaves;
+    // The item's partial rows and LSEs, from its first segment on (byte
+    // offsets fit 32 bits: n segments of NO floats).
+    const __amdgpu_buffer_rsrc_t rs =
+        buffer_rsrc(p.partial_out + static_cast<size_t>(it.s0) * NO, it.n * NO * static_cast<int>(sizeof(float)));
+    const __amdgpu_buffer_rsrc_t rl =
+        buffer_rsrc(p.partial_lse + static_cast<size_t>(it.s0) * G, it.n * G * static_cast<int>(sizeof(float)));
+    float m[S], den[S];
+    f32x4 acc[S];
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        m[s]   = -INFINITY;
+        den[s] = 0.f;
+        acc[s] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    for (int jb = j0; jb <= j1; jb += NGR * U) {
+        u32x4 raw[S][U];
+        float ls[S][U];
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+#pragma unroll
+            for (int k = 0; k < U; ++k) {
+                const int j = jb + S * li + s + NGR * k;
+                if (j <= j1) {
+                    const int sg = max(0, kWaves * j - it.u0);   // the block's first segment, from s0
+                    raw[s][k] = __builtin_bit_cast(
+                        u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                   rs, (sg * NO + 4 * vi) * static_cast<int>(sizeof(float)), 0, kAuxCoherent));
+                    ls[s][k] = __builtin_bit_cast(
+                        float, __builtin_amdgcn_raw_buffer_load_b32(
+                                   rl, (sg * G + hh) * static_cast<int>(sizeof(float)), 0, kAuxCoherent));
+                }
+            }
+#if PA_STAMPS
+        __builtin_amdgcn_s_waitcnt(kWaitVm0);
+        if (t == 0 && jb == j0) stamp(12);
+#endif
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+#pragma unroll
+            for (int k = 0; k < U; ++k) {
+                if (jb + S * li + s + NGR * k > j1) break;
+                const float mn  = fmaxf(m[s], ls[s][k]);
+                const float f   = exp2_fast(m[s] - mn);   // 0 while m = -inf
+                const float wgt = exp2_fast(ls[s][k] - mn);
+                const f32x4 v   = __builtin_bit_cast(f32x4, raw[s][k]);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) acc[s][c] = fmaf(wgt, v[c], acc[s][c] * f);
+                den[s] = fmaf(den[s], f, wgt);
+                m[s]   = mn;
+            }
+    }
+    // The tree (a state with no block has m = -inf and weighs 0).
+    auto combine = [&](float m2, float d2, const f32x4& a2) {
+        const float mt = fmaxf(m[0], m2);
+        const float f1 = m[0] == -INFINITY ? 0.f : exp2_fast(m[0] - mt);
+        const float f2 = m2 == -INFINITY ? 0.f : exp2_fast(m2 - mt);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) acc[0][c] = acc[0][c] * f1 + a2[c] * f2;
+        den[0] = den[0] * f1 + d2 * f2;
+        m[0]   = mt;
+    };
+    auto partner_round = [&](auto ctrl) {
+        constexpr int C = decltype(ctrl)::value;
+        f32x4 a2;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) a2[c] = dpp_f32<C>(acc[0][c]);
+        combine(dpp_f32<C>(m[0]), dpp_f32<C>(den[0]), a2);
+    };
+    if (t == 0) stamp(13);
+    // A round whose partners hold no block changes nothing and is left out.
+    const int nb = j1 - j0 + 1;
+    if constexpr (S == 2) combine(m[1], den[1], acc[1]);
+    if constexpr (LPV >= 2)
+        if (nb > S) partner_round(std::integral_constant<int, 0xB1>{});        // quad_perm [1,0,3,2]
+    if constexpr (LPV >= 4)
+        if (nb > 2 * S) partner_round(std::integral_constant<int, 0x4E>{});    // quad_perm [2,3,0,1]
+    if constexpr (LPV >= 8)
+        if (nb > 4 * S) partner_round(std::integral_constant<int, 0x141>{});   // row_half_mirror
+    if constexpr (LPV >= 16)
+        if (nb > 8 * S) partner_round(std::integral_constant<int, 0x140>{});   // row_mirror
+    if (t == 0) stamp(14);
+    if (li == 0) {
+        const float inv = 1.0f / den[0];
+        const f16x2 lo = {static_cast<_Float16>(acc[0][0] * inv), static_cast<_Float16>(acc[0][1] * inv)};
+        const f16x2 hi = {static_cast<_Float16>(acc[0][2] * inv), static_cast<_Float16>(acc[0][3] * inv)};
+        *reinterpret_cast<u32x2*>(p.out + static_cast<size_t>(it.item) * NO + 4 * vi) =
+            u32x2{__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi)};
+    }
+    if (t == 0) stamp(15);
+}
+
+// Block-level merge after the split loop. `slots` holds, per wave, its first
+// (slot 0) and last (slot 1) segment when that segment is a split one; part /
+// lse hold the slot's normalized partial rows and base-2 LSEs, written to LDS
+// by the wave that computed them. The slots of one item are a run of the
+// filled slots: a run starts at an item's first segment, or at the block's
+// first filled slot (an item continued from the previous block). The result
+// is the base-2 LSE-weighted average of a run's partials
+// (decode_kernels.cuh:409-432), summed in slot order.
+//
+// Bound by the latency of one run's chain (LDS reads, exponentials, division,
+// store: 0.7 us by stamps), not by throughput. So the work is cut into tasks of
+// 256 elements (4 per lane) of one run, task t on wave t mod 8, and the runs of
+// a block are merged side by side: ragged batches have 3 to 9 runs in a block,
+// which took 0.5 us each after the block's last wave when every thread did one
+// element of every run in turn. Same box, us per step, before and after: 37
+// ragged FP8 rows of up to 3001 tokens 23.7 -> 20.7 (64 query heads, 24-token
+// pages: 28.6 -> 23.8), 32 rows of 200 12.0 -> 10.0, 128 rows of 16 to 1000
+// 48.3 -> 44.8, 1 row of 200 8.5 -> 7.0; one run in every block (4 x 1024,
+// 32 x 1024) is level. Eight elements per lane (half the tasks) were 0.3 us
+// slower where a block holds one or two runs and no faster elsewhere.
 //
 // An item whose segments all lie in this block (block_merge 1: every split
 // item) is written as fp16. With block_merge 2 an item may also span blocks
@@ -334,88 +474,115 @@ __device__ __forceinline__ void store_coherent(float* p, float v) {
 // the merge kernel does (so the result does not depend on which block is
 // last). Blocks never wait for each other.
 template <int G>
-__device__ __forceinline__ void block_merge(const pa_decode_params& p, const int32_t* __restrict__ isb,
-                                            const int (*slot_item)[2], const int (*slot_seg)[2],
+__device__ __forceinline__ void block_merge(const pa_decode_params& p, const Slot* slots,
                                             const float (*part)[G * kHeadDim], const float (*lse)[G],
                                             int* last_lds, int tid, int lblock) {
-    constexpr int NS = 2 * kWaves;
-    constexpr int NO = G * kHeadDim;
-    constexpr int NE = (NO + 64 * kWaves - 1) / (64 * kWaves);   // elements per thread
-    static_assert(NS == 16, "the slot lanes form one DPP row");
-    static_assert(kHeadDim % 64 == 0, "a wave's elements share one head");
+    constexpr int NS  = 2 * kWaves;
+    constexpr int NO  = G * kHeadDim;
+    constexpr int TPR = NO > 256 ? NO / 256 : 1;   // tasks per run
+    static_assert(NS == 16, "the slots fit the low lanes of a wave");
     const int  lane  = tid & 63;
-    const bool slot  = lane < NS;   // lane j holds slot j
+    const int  wave  = __builtin_amdgcn_readfirstlane(tid >> 6);
     const bool chain = p.block_merge == 2;
     if (tid == 0) stamp(16);
-    float lv[NE], pv[NE][NS];
-#pragma unroll
-    for (int e = 0; e < NE; ++e) {
-        const int o = tid + 64 * kWaves * e;
-        if (o < NO) {
-            lv[e] = lse[lane & (NS - 1)][o / kHeadDim];
-#pragma unroll
-            for (int j = 0; j < NS; ++j) pv[e][j] = part[j][o];
-        }
-    }
-    const int      mine   = slot_item[(lane & (NS - 1)) >> 1][lane & 1];
-    const int      myseg  = slot_seg[(lane & (NS - 1)) >> 1][lane & 1];
+    const Slot     mine   = slots[lane & (NS - 1)];   // lane j holds slot j
+    const uint32_t filled = static_cast<uint32_t>(__builtin_amdgcn_ballot_w64(lane < NS && mine.item >= 0));
+    if (filled == 0) return;
+    const uint32_t starts = static_cast<uint32_t>(__builtin_amdgcn_ballot_w64(
+        lane < NS && mine.item >= 0 && (mine.seg == mine.s0 || lane == __builtin_ctz(filled))));
 #if PA_STAMPS
-    __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
     if (tid == 0) stamp(17);
 #endif
-    const uint64_t filled = __builtin_amdgcn_ballot_w64(slot && mine >= 0);
-    // Items of this block that span blocks (at most two), block-uniform.
-    int ns = 0, sx0 = 0, su0 = 0, sn0 = 0, sx1 = 0, su1 = 0, sn1 = 0;
-    uint64_t run = 0;
-    for (uint64_t rem = filled; rem != 0; rem &= ~run) {
-        const int j0 = __builtin_ctzll(rem);
-        const int x  = __builtin_amdgcn_readlane(mine, j0);   // the next item
-        run = __builtin_amdgcn_ballot_w64(slot && mine == x);
-        const int  n     = isb[x + 1] - isb[x];
-        const bool spans = chain && __builtin_popcountll(run) != n;
+    // The run whose first slot is the lowest bit of `from` (a suffix of starts).
+    auto run_of = [&](uint32_t from) {
+        const uint32_t next = from & (from - 1);                        // the following run's start
+        const uint32_t upto = next ? (next & (0u - next)) - 1u : ~0u;   // the slots before it
+        return filled & upto & ~((from & (0u - from)) - 1u);
+    };
+    const int runs = __builtin_popcount(starts);
+    for (int t = wave; t < runs * TPR; t += kWaves) {
+        uint32_t from = starts;
+        for (int r = t / TPR; r > 0; --r) from &= from - 1;
+        const uint32_t run  = run_of(from);
+        const int  j0    = __builtin_ctz(from);
+        const int  item  = __builtin_amdgcn_readlane(mine.item, j0);
+        const int  bseg  = __builtin_amdgcn_readlane(mine.seg, j0);   // the item's first segment here
+        const int  n     = __builtin_amdgcn_readlane(mine.n, j0);
+        const bool spans = chain && __builtin_popcount(run) != n;
 #if PA_STAMPS
-        if (tid == 0 && rem == filled) stamp(18 + spans);
+        if (tid == 0 && t == 0) stamp(18 + spans);
 #endif
-        const int  bseg  = __builtin_amdgcn_readlane(myseg, j0);   // the item's first segment here
-        if (spans) {
-            const int u0 = lblock * kWaves + (j0 >> 1) - (bseg - isb[x]);   // unit of its first segment
-            if (ns == 0) { sx0 = x; su0 = u0; sn0 = n; }
-            else { sx1 = x; su1 = u0; sn1 = n; }
-            ++ns;
-        }
-        const bool in = (run >> lane) & 1;
+        const int o = 256 * (t % TPR) + 4 * lane;
+        if (NO >= 256 || o < NO) {
+            const int hd = o / kHeadDim;
+            float mx = -INFINITY, den = 0.f;
+            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+            // Eight slots at a time (every plan of make_plan's has at most
+            // eight in a run): all their LDS reads, then the weights. Past
+            // the run's end nothing is read and the weight is 0.
+            for (uint32_t rem = run; rem != 0;) {
+                float ls[8];
+                f32x4 v[8];
 #pragma unroll
-        for (int e = 0; e < NE; ++e) {
-            const int o = tid + 64 * kWaves * e;
-            if (o >= NO) break;
-            // The item's maximum LSE over the 16 slot lanes (one DPP row):
-            // swaps of neighbours and pairs in each quad, then rotations by 4
-            // and 8.
-            float mx = in ? lv[e] : -INFINITY;
-            mx = fmaxf(mx, dpp_f32<0xB1>(mx));    // quad_perm [1,0,3,2]
-            mx = fmaxf(mx, dpp_f32<0x4E>(mx));    // quad_perm [2,3,0,1]
-            mx = fmaxf(mx, dpp_f32<0x124>(mx));   // row_ror:4
-            mx = fmaxf(mx, dpp_f32<0x128>(mx));   // row_ror:8
-            const float w = in ? exp2_fast(lv[e] - mx) : 0.f;
-            float a = 0.f, den = 0.f;
+                for (int k = 0; k < 8; ++k) {
+                    ls[k] = -INFINITY;
+                    v[k]  = f32x4{0.f, 0.f, 0.f, 0.f};
+                    if (rem) {
+                        const int j = __builtin_ctz(rem);
+                        rem &= rem - 1;
+                        ls[k] = lse[j][hd];
+                        v[k]  = *reinterpret_cast<const f32x4*>(&part[j][o]);
+                    }
+                }
+                float mn = mx;
 #pragma unroll
-            for (int j = 0; j < NS; ++j) {
-                const float wj = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), j));
-                a   = fmaf(wj, ((run >> j) & 1) ? pv[e][j] : 0.f, a);   // empty slots hold no partial
-                den = den + wj;
+                for (int k = 0; k < 8; ++k) mn = fmaxf(mn, ls[k]);
+                const float f = exp2_fast(mx - mn);   // 0 at the first eight
+                den *= f;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) acc[c] *= f;
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    const float w = exp2_fast(ls[k] - mn);
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) acc[c] = fmaf(w, v[k][c], acc[c]);
+                    den += w;
+                }
+                mx = mn;
             }
+            const float inv = 1.0f / den;
             if (!spans) {
-                const int b = x / p.num_kv_heads, h = x - b * p.num_kv_heads;
-                p.out[(static_cast<size_t>(b) * p.num_q_heads + h * G) * kHeadDim + o] =
-                    __builtin_bit_cast(uint16_t, static_cast<_Float16>(a * (1.0f / den)));
+                const f16x2 lo = {static_cast<_Float16>(acc[0] * inv), static_cast<_Float16>(acc[1] * inv)};
+                const f16x2 hi = {static_cast<_Float16>(acc[2] * inv), static_cast<_Float16>(acc[3] * inv)};
+                *reinterpret_cast<u32x2*>(p.out + static_cast<size_t>(item) * NO + o) =
+                    u32x2{__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi)};
             } else {
-                store_coherent(p.partial_out + static_cast<size_t>(bseg) * NO + o, a * (1.0f / den));
+                const __amdgpu_buffer_rsrc_t rs = buffer_rsrc(p.partial_out + static_cast<size_t>(bseg) * NO,
+                                                              NO * static_cast<int>(sizeof(float)));
+                store_coherent16(rs, o * static_cast<int>(sizeof(float)),
+                                 f32x4{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv});
                 if (o % kHeadDim == 0)
-                    store_coherent(p.partial_lse + static_cast<size_t>(bseg) * G + o / kHeadDim, mx + __log2f(den));
+                    store_coherent(p.partial_lse + static_cast<size_t>(bseg) * G + hd, mx + __log2f(den));
             }
         }
     }
-    if (ns == 0) return;
+    if (!chain) return;
+    // Items of this block that span blocks: its first run, its last, or both
+    // (sa; sb when there are two).
+    auto span_of = [&](uint32_t from) {
+        const int j0 = __builtin_ctz(from);
+        const int s0 = __builtin_amdgcn_readlane(mine.s0, j0);
+        const int u0 = lblock * kWaves + (j0 >> 1) - (__builtin_amdgcn_readlane(mine.seg, j0) - s0);
+        return Span{__builtin_amdgcn_readlane(mine.item, j0), s0, __builtin_amdgcn_readlane(mine.n, j0), u0};
+    };
+    const uint32_t last_start = 1u << (31 - __builtin_clz(starts));
+    const Span     first_run  = span_of(starts), last_run = span_of(last_start);
+    const bool     first_spans = __builtin_popcount(run_of(starts)) != first_run.n;
+    const bool     last_spans  = runs > 1 && __builtin_popcount(run_of(last_start)) != last_run.n;
+    if (!first_spans && !last_spans) return;
+    const int  ns = first_spans && last_spans ? 2 : 1;
+    const Span sa = first_spans ? first_run : last_run;
+    const Span sb = last_run;
     if (tid == 0) stamp(9);
 
     // Arrivals: this block's partial rows are complete at the coherence point
@@ -424,11 +591,9 @@ __device__ __forceinline__ void block_merge(const pa_decode_params& p, const int
     __syncthreads();
     if (tid == 0) stamp(10);
     if (tid < ns) {
-        const int x  = tid == 0 ? sx0 : sx1;
-        const int u0 = tid == 0 ? su0 : su1;
-        const int n  = tid == 0 ? sn0 : sn1;
-        const int nb = (u0 + n - 1) / kWaves - u0 / kWaves + 1;   // blocks the item spans
-        int* ctr = p.merge_counters + x;
+        const Span it = tid == 0 ? sa : sb;
+        const int  nb = (it.u0 + it.n - 1) / kWaves - it.u0 / kWaves + 1;   // blocks the item spans
+        int* ctr = p.merge_counters + it.item;
         const int before = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         const bool last = before == nb - 1;
         if (last) __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // for the next decode
@@ -436,105 +601,12 @@ __device__ __forceinline__ void block_merge(const pa_decode_params& p, const int
     }
     __syncthreads();
     if (tid == 0) stamp(11);
-    // The last block combines the item's block partials (block j's sits at the
-    // item's first segment in block j). Thread (v, g), g = tid % NGR, takes
-    // 16 bytes (4 dims) v of every NGR-th block from g on, up to 8 blocks at a
-    // time, each with one coherent 16-byte load of the row and one of its LSE,
-    // all issued before the first is used (one round trip), and keeps a
-    // running maximum over them in block order; the NGR states of one dim
-    // vector sit in adjacent lanes of one DPP row and are combined in a fixed
-    // tree (lanes 1, 2 apart, then quad and half-row mirrors), so the result
-    // does not depend on timing.
-    constexpr int NV  = NO / 4;                  // 16-byte vectors of one block partial
-    constexpr int NGR = 64 * kWaves / NV;        // lanes sharing one vector (16, 8, 4, 2 for G = 1, 2, 4, 8)
-    static_assert(NGR >= 1 && NGR <= 16 && (NGR & (NGR - 1)) == 0, "the groups of a vector form one DPP row");
-    const int gi = tid % NGR;
-    const int vi = tid / NGR;
-    const int hh = 4 * vi / kHeadDim;            // query head of the vector
-    for (int i = 0; i < ns; ++i) {
-        if (!last_lds[i]) continue;
-        const int x  = i == 0 ? sx0 : sx1;
-        const int u0 = i == 0 ? su0 : su1;
-        const int n  = i == 0 ? sn0 : sn1;
-        const int s0 = isb[x];
-        const int j0 = u0 / kWaves, j1 = (u0 + n - 1) / kWaves;
-        const int nb = j1 - j0 + 1;
-        const int b = x / p.num_kv_heads, h = x - b * p.num_kv_heads;
-        // The item's partial rows and LSEs, from its first segment on (byte
-        // offsets fit 32 bits: n segments of NO floats).
-        const __amdgpu_buffer_rsrc_t rs =
-            buffer_rsrc(p.partial_out + static_cast<size_t>(s0) * NO, n * NO * static_cast<int>(sizeof(float)));
-        const __amdgpu_buffer_rsrc_t rl =
-            buffer_rsrc(p.partial_lse + static_cast<size_t>(s0) * G, n * G * static_cast<int>(sizeof(float)));
-        float  m = -INFINITY, den = 0.f;
-        f32x4  acc = {0.f, 0.f, 0.f, 0.f};
-        const int per = (nb + NGR - 1) / NGR;   // blocks per group (the first groups may take one more)
-        for (int k0 = 0; k0 < per; k0 += 8) {
-            u32x4 raw[8];
-            float ls[8];
-#pragma unroll
-            for (int t = 0; t < 8; ++t) {
-                const int j = j0 + gi + NGR * (k0 + t);
-                if (j <= j1) {
-                    const int k = max(0, kWaves * j - u0);   // the block's first segment, from s0
-                    raw[t] = __builtin_bit_cast(
-                        u32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                   rs, (k * NO + 4 * vi) * static_cast<int>(sizeof(float)), 0, kAuxCoherent));
-                    ls[t] = __builtin_bit_cast(
-                        float, __builtin_amdgcn_raw_buffer_load_b32(
-                                   rl, (k * G + hh) * static_cast<int>(sizeof(float)), 0, kAuxCoherent));
-                }
-            }
-#if PA_STAMPS
-            __builtin_amdgcn_s_waitcnt(kWaitVm0);
-            if (tid == 0 && i == 0 && k0 == 0) stamp(12);
-#endif
-#pragma unroll
-            for (int t = 0; t < 8; ++t) {
-                const int j = j0 + gi + NGR * (k0 + t);
-                if (j > j1) break;
-                const float mn  = fmaxf(m, ls[t]);
-                const float f   = exp2_fast(m - mn);   // 0 while m = -inf
-                const float wgt = exp2_fast(ls[t] - mn);
-                const f32x4 v   = __builtin_bit_cast(f32x4, raw[t]);
-#pragma unroll
-                for (int c = 0; c < 4; ++c) acc[c] = fmaf(wgt, v[c], acc[c] * f);
-                den = fmaf(den, f, wgt);
-                m   = mn;
-            }
-        }
-        // Combine the NGR states of the vector (a group with no block has
-        // m = -inf and weighs 0).
-        auto combine = [&](float m2, float d2, const f32x4& a2) {
-            const float mt = fmaxf(m, m2);
-            const float f1 = m == -INFINITY ? 0.f : exp2_fast(m - mt);
-            const float f2 = m2 == -INFINITY ? 0.f : exp2_fast(m2 - mt);
-#pragma unroll
-            for (int c = 0; c < 4; ++c) acc[c] = acc[c] * f1 + a2[c] * f2;
-            den = den * f1 + d2 * f2;
-            m   = mt;
-        };
-        auto partner_round = [&](auto ctrl) {
-            constexpr int C = decltype(ctrl)::value;
-            f32x4 a2;
-#pragma unroll
-            for (int c = 0; c < 4; ++c) a2[c] = dpp_f32<C>(acc[c]);
-            combine(dpp_f32<C>(m), dpp_f32<C>(den), a2);
-        };
-        if (tid == 0 && i == 0) stamp(13);
-        if constexpr (NGR >= 2) partner_round(std::integral_constant<int, 0xB1>{});    // quad_perm [1,0,3,2]
-        if constexpr (NGR >= 4) partner_round(std::integral_constant<int, 0x4E>{});    // quad_perm [2,3,0,1]
-        if constexpr (NGR >= 8) partner_round(std::integral_constant<int, 0x141>{});   // row_half_mirror
-        if constexpr (NGR >= 16) partner_round(std::integral_constant<int, 0x140>{});  // row_mirror
-        if (tid == 0 && i == 0) stamp(14);
-        if (gi == 0) {
-            const float inv = 1.0f / den;
-            const f16x2 lo = {static_cast<_Float16>(acc[0] * inv), static_cast<_Float16>(acc[1] * inv)};
-            const f16x2 hi = {static_cast<_Float16>(acc[2] * inv), static_cast<_Float16>(acc[3] * inv)};
-            *reinterpret_cast<u32x2*>(p.out + (static_cast<size_t>(b) * p.num_q_heads + h * G) * kHeadDim + 4 * vi) =
-                u32x2{__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi)};
-        }
-        if (tid == 0 && i == 0) stamp(15);
+    const bool last_a = last_lds[0] != 0, last_b = ns > 1 && last_lds[1] != 0;
+    if (last_a && last_b) {
+        const bool lower = wave < kWaves / 2;
+        combine_blocks<G, 2>(p, lower ? sa : sb, lower ? tid : tid - 32 * kWaves);
+    } else if (last_a || last_b) {
+        combine_blocks<G, 1>(p, last_a ? sa : sb, tid);
     }
 }
 
@@ -578,8 +650,7 @@ __device__ __forceinline__ void decode_split_body(const pa_decode_params& p, con
     // Compact Q per wave (G heads x 256 B; on the LDS-destination paths filled
     // by issue() with the K / V, 1 KiB per load).
     __shared__ __attribute__((aligned(16))) u32x4 q_lds[kWaves][64 * NQ];
-    __shared__ int slot_item[kWaves][2];                                     // split segments per wave
-    __shared__ int slot_seg[kWaves][2];                                      // their segment indices
+    __shared__ Slot slots[2 * kWaves];                                       // split segments, 2 * wave + sl
     __shared__ int last_lds[2];                                              // block merges a spanning item
     // LDS stage of one step per wave (STG): [K, V][half][16 rows][row bytes],
     // each row's 16-byte chunks XOR-swizzled by (row % chunks per row).
@@ -598,8 +669,8 @@ __device__ __forceinline__ void decode_split_body(const pa_decode_params& p, con
     const int unit   = lblock * kWaves + wave;
     const bool merge_here = p.block_merge != 0;   // block-level merge of split rows
     if (lane == 0) {
-        slot_item[wave][0] = -1;
-        slot_item[wave][1] = -1;
+        slots[2 * wave].item     = -1;
+        slots[2 * wave + 1].item = -1;
     }
     int seg_begin = 0, seg_end = 0;
     if (unit < num_units) {
@@ -873,6 +944,7 @@ __device__ __forceinline__ void decode_split_body(const pa_decode_params& p, con
     f32x4 oacc[8];    // O[head 4kb+i][dim 8c+j] = oacc[j][i]
     float m_run = -INFINITY, l_run = 0.f;
     bool  whole = false;
+    int   item_s0 = 0, item_n = 0;   // the item's first segment and segment count
 #pragma unroll
     for (int j = 0; j < 8; ++j) oacc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
@@ -920,10 +992,7 @@ __device__ __forceinline__ void decode_split_body(const pa_decode_params& p, con
                         if (c == 0) p.partial_lse[static_cast<size_t>(C.seg) * G + 4 * kb + i] = ls;
                     }
                 }
-                if (merge_here && lane == 0) {
-                    slot_item[wave][sl] = C.b * hkv + C.h;
-                    slot_seg[wave][sl]  = C.seg;
-                }
+                if (merge_here && lane == 0) slots[2 * wave + sl] = Slot{C.b * hkv + C.h, C.seg, item_s0, item_n};
             }
         }
         m_run = -INFINITY;
@@ -974,7 +1043,9 @@ __device__ __forceinline__ void decode_split_body(const pa_decode_params& p, con
 #pragma unroll
             for (int j = 0; j < 4; ++j) qf[j] = ql[16 * hc + (KNAT ? 4 * j + kb : 4 * kb + j)];
             const int item = C.b * hkv + C.h;
-            whole = isb[item + 1] - isb[item] == 1;
+            item_s0 = isb[item];
+            item_n  = isb[item + 1] - item_s0;
+            whole   = item_n == 1;
         }
         if constexpr (STG) {
             // Coalesced rows -> LDS (16-byte chunk j of row r at chunk j ^ (r % CPR))
@@ -1182,7 +1253,7 @@ __device__ __forceinline__ void decode_split_body(const pa_decode_params& p, con
 
     if (merge_here) {
         __syncthreads();
-        block_merge<G>(p, isb, slot_item, slot_seg, part_lds, lse_lds, last_lds, threadIdx.x, lblock);
+        block_merge<G>(p, slots, part_lds, lse_lds, last_lds, threadIdx.x, lblock);
     }
 }
 

@@ -22,9 +22,9 @@ One JSON line per shape:
   merge_in_block     per block, from its last wave's end to its merged items
                      (the LDS merge, and for items that span blocks the
                      partial row stored), then its parts: barrier (to the
-                     merge's start), lds (the slots' partials read),
-                     count (the first item's segment count loaded), average
-                     (the weighted average computed, its stores issued)
+                     merge's start), lds (the slots' items read), count (wave
+                     0's first task found), average (wave 0's tasks: partials
+                     read, weighted average computed, its stores issued)
   store_wait         those partial rows complete at the coherence point
   arrive             the arrival counter's round trip
   combine            the last block's combine of an item's block partials:

@@ -1,0 +1,92 @@
+"""The split kernel's merges where a block holds many split rows, a run of more
+than eight slots, or two rows that it is the last block of: against the merge
+kernel on the same plan and the fp32 oracle, and bitwise equal from run to run.
+"""
+
+from __future__ import annotations
+
+import ctypes
+
+import numpy as np
+import pytest
+
+import oracle
+import pa_amd
+from helpers import D, TOL, paged_inputs
+
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("gpu_device")]
+
+
+def _check(fp8, lens, group, hkv, handle, mode, page=16, repeats=6):
+    import torch
+    hq = hkv * group
+    dt = pa_amd.FP8_E4M3 if fp8 else pa_amd.FP16
+    q, k, v, table, ks, vs = paged_inputs(len(lens), lens, hq, hkv, page, fp8, seed=7 * group + len(lens))
+    dplan = pa_amd.DevicePlan()
+    pa_amd._lib.call("pa_device_plan_upload", dplan._h, handle, group, D, None)
+    outs = []
+    for rep in range(repeats + 1):
+        p = pa_amd.DecodeParams()
+        p.q, p.k_cache, p.v_cache, p.block_table = q.data_ptr(), k.data_ptr(), v.data_ptr(), table.data_ptr()
+        out = torch.full_like(q, float("nan"))
+        p.out = out.data_ptr()
+        p.block_table_stride = table.size(1)
+        p.batch, p.num_q_heads, p.num_kv_heads, p.head_dim, p.page_size = len(lens), hq, hkv, D, page
+        p.sm_scale, p.k_scale, p.v_scale = pa_amd.sm_scale(D), ks, vs
+        dplan.bind(p)
+        assert p.block_merge == mode and p.needs_merge == 0
+        if rep == repeats:
+            p.block_merge, p.needs_merge = 0, 1   # the merge kernel on the same plan
+        pa_amd.paged_decode(dt, p)
+        torch.cuda.synchronize()
+        outs.append(out)
+    for o in outs[1:repeats]:
+        assert torch.equal(outs[0].view(torch.int16), o.view(torch.int16))
+    kb = k.view(torch.uint8).cpu().numpy() if fp8 else k.view(torch.int16).cpu().numpy().view(np.uint16)
+    vb = v.view(torch.uint8).cpu().numpy() if fp8 else v.view(torch.int16).cpu().numpy().view(np.uint16)
+    ref = oracle.paged_decode(dt, q.view(torch.int16).cpu().numpy().view(np.uint16), kb, vb, table.cpu().numpy(),
+                              np.asarray(lens, np.int32), hq, hkv, D, page, ks, vs, threads=16)
+    for o in (outs[0], outs[-1]):
+        assert float(np.max(np.abs(o.float().cpu().numpy() - ref))) < TOL
+    # Both merges average the same fp32 partials; two fp16 roundings of values below 4 differ by at most 2^-9.
+    assert float((outs[0].float() - outs[-1].float()).abs().max()) <= 2.0 ** -9
+
+
+def _plan(fp8, lens, group, hkv, ctas):
+    return pa_amd.make_plan(pa_amd.FP8_E4M3 if fp8 else pa_amd.FP16, lens, hkv * group, hkv, D, ctas)
+
+
+@pytest.mark.parametrize("group", [1, 2, 4, 8])
+@pytest.mark.parametrize("fp8", [False, True], ids=["fp16", "fp8"])
+def test_many_split_rows_in_a_block(fp8, group):
+    """Rows of 2 to 5 tiles over units of 3: most blocks hold 5 to 9 runs, the first and last of them
+    continuing in the neighbouring blocks, so a block is often the last of two rows at once."""
+    tile = 32 if fp8 else 16
+    rng = np.random.default_rng(3)
+    lens = [int(x) for x in rng.integers(tile + 1, 5 * tile, size=40)]
+    total = sum(-(-n // tile) for n in lens) * 8
+    plan = _plan(fp8, lens, group, 8, -(-total // 3))
+    _check(fp8, lens, group, 8, plan.handle.value, 2)
+
+
+@pytest.mark.parametrize("lens,ctas", [([100], 0), ([129], 0), ([16 * 17] * 3, 0), ([5000, 1, 700, 16, 17], 96)],
+                         ids=["7_tiles", "9_tiles", "17_tiles", "mixed"])
+def test_short_rows_across_blocks(lens, ctas):
+    """Rows that straddle two or three blocks because their tiles are no multiple of a block's units."""
+    plan = _plan(False, lens, 4, 8, ctas)
+    _check(False, lens, 4, 8, plan.handle.value, 2)
+
+
+@pytest.mark.parametrize("group", [1, 4, 8])
+def test_run_of_sixteen_slots(group):
+    """A caller's plan that gives every unit of a block two segments of one row: 16 slots in one run."""
+    segs = np.array([[0, 0, 16 * i, 16 * i + 16] for i in range(16)] + [[1, 0, 0, 16], [1, 0, 16, 29]], np.int32)
+    cta = np.array([0, 2, 4, 6, 8, 10, 12, 14, 16, 17, 18], np.int32)
+    item = np.array([0, 16, 18], np.int32)
+    h = ctypes.c_void_p()
+    pa_amd._lib.call("pa_plan_create", 10, 16, segs.ctypes.data, len(segs), cta.ctypes.data, item.ctypes.data, 2, 1,
+                     ctypes.byref(h))
+    try:
+        _check(False, [256, 29], group, 1, h.value, 1)
+    finally:
+        pa_amd._lib.load().pa_plan_destroy(h.value)
