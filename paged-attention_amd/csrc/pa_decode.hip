@@ -38,7 +38,7 @@
 //     and every slot issues the same loads, which keeps the hardware wait
 //     counts exact. Smaller
 //     pages go through the LDS stage for both element types: pages of whole
-//     1 KiB parts (fp16 P = 4 and 8, FP8 P = 8) with one resource per part,
+//     1 KiB parts (fp16 multiples of 4 tokens, FP8 of 8) with one resource per part,
 //     any other size with each lane loading a row whose page it looks up
 //     itself (the step's table entries spread over the lanes, handed out by
 //     ds_bpermute).
@@ -219,9 +219,25 @@ enum PagePath : int {
                      // token, integer division
     kPageRuns = 3,   // page_size 4 or 8 (fp16) / 8 (FP8 with the LDS stage): K/V through
                      // the LDS stage, one wave-uniform page per coalesced 1 KiB part
-    kPageLane = 4,   // every other page size (1, 2, FP8 4, any non-power of two): K/V
+    kPageLane = 4,   // every other page size (1, 2, FP8 4, odd sizes): K/V
                      // through the LDS stage, each lane finding the page of the row it
                      // loads (coalesced 16-byte loads at per-lane addresses)
+    kPageRunsDiv = 5,   // kPageRuns for page sizes that are multiples of a 1 KiB part's rows but
+                        // no powers of two (a part starts on a multiple of its rows, so it
+                        // lies in one page): the page by division, see PageDiv
+};
+
+// tok / page_size and what is left, without a divide: a shift for powers of
+// two (shift >= 0), else floor(tok * magic / 2^(31 + l)) with l = ceil(log2 P)
+// and magic = floor(2^(31 + l) / P) + 1, stored as shift = ~(l - 1). Exact for
+// 0 <= tok < 2^31: with r = tok mod P, tok * magic / 2^(31 + l) = tok / P + e and
+// 0 < e <= tok / 2^(31 + l) < 2^-l <= 1 / P, so adding e to r / P <= (P - 1) / P stays below 1.
+struct PageDiv {
+    int      shift;
+    uint32_t magic;
+    __device__ __forceinline__ int page(int tok) const {
+        return shift >= 0 ? tok >> shift : static_cast<int>(__umulhi(static_cast<uint32_t>(tok), magic) >> ~shift);
+    }
 };
 
 // One position of a wave's schedule: the current step of the current segment.
@@ -619,7 +635,7 @@ __device__ __forceinline__ void block_merge(const pa_decode_params& p, const Slo
 //   PATH  page resolution (PagePath)
 template <int EB, int G, int NG, int DEPTH, int PATH>
 __device__ __forceinline__ void decode_split_body(const pa_decode_params& p, const int32_t* __restrict__ cta,
-                                                  int num_units, int page_shift,
+                                                  int num_units, const PageDiv pd,
                                                   const int32_t* __restrict__ tbl, const int32_t* __restrict__ sid,
                                                   const int32_t* __restrict__ segp, const int32_t* __restrict__ isb) {
     constexpr int  NH    = NG / 16;                 // 16-token halves per step
@@ -634,7 +650,8 @@ __device__ __forceinline__ void decode_split_body(const pa_decode_params& p, con
     constexpr int  NQ    = G > 4 ? 2 : 1;           // compact Q registers per lane
     constexpr int  NVL   = PATH == kPageAny ? 4 : 1;   // V page lookups per lane (per-lane paths)
     constexpr int  HW    = G < 4 ? G : 4;           // live O rows per writing lane
-    constexpr bool STG   = PATH == kPageRuns || PATH == kPageLane ||
+    constexpr bool RUNS  = PATH == kPageRuns || PATH == kPageRunsDiv;
+    constexpr bool STG   = RUNS || PATH == kPageLane ||
                            (Tune<EB>::stage && PATH == kPagePow2);   // K/V via LDS
     constexpr int  RPP   = 1024 / ROW;              // rows per coalesced 1 KiB part (4 fp16, 8 FP8)
     constexpr int  NPART = 16 / RPP;                // parts per 16-token half
@@ -710,7 +727,7 @@ __device__ __forceinline__ void decode_split_body(const pa_decode_params& p, con
     u32x4 kc[STG && !DMA ? DEPTH : 1][NH][NPART], vc[STG && !DMA ? DEPTH : 1][NH][NPART];
     u32x4 qc[DMA ? 1 : DEPTH][NQ];   // compact Q, loaded with a segment's first step (direct paths)
     int   pg[DEPTH][NH];       // power-of-two path: page of each half (wave-uniform)
-    int   pgr[PATH == kPageRuns ? DEPTH : 1][NH][NPART];   // small pages: page of each part
+    int   pgr[RUNS ? DEPTH : 1][NH][NPART];   // page of each part
     constexpr int LN = PATH == kPageLane ? DEPTH : 1;
     int   plk[LN][NH][NPART], psl[LN][NH][NPART];          // lane path: byte address of the lane holding
                                                            // the row's page entry, slot in the page
@@ -726,21 +743,25 @@ __device__ __forceinline__ void decode_split_body(const pa_decode_params& p, con
     const int* t_row = table_row(p, tbl, sid, T.b);
     bool t_more = true, l_more = true;
 
+    // The page of a 1 KiB part's first token (page-run paths).
+    auto part_page = [&](int tok) { return PATH == kPageRunsDiv ? pd.page(tok) : tok >> pd.shift; };
+    auto part_slot = [&](int tok) { return PATH == kPageRunsDiv ? tok - pd.page(tok) * P : tok & (P - 1); };
+
     // Page lookups of step T into slot s, then advance T.
     auto lookup = [&](int s) {
         if constexpr (PATH == kPagePow2) {
             if (t_more) {
 #pragma unroll
                 for (int hh = 0; hh < NH; ++hh)
-                    pg[s][hh] = load_uniform(t_row, min(T.tok + 16 * hh, T.w - 1) >> page_shift);
+                    pg[s][hh] = load_uniform(t_row, min(T.tok + 16 * hh, T.w - 1) >> pd.shift);
             }
-        } else if constexpr (PATH == kPageRuns) {
+        } else if constexpr (RUNS) {
             if (t_more) {
 #pragma unroll
                 for (int hh = 0; hh < NH; ++hh)
 #pragma unroll
                     for (int part = 0; part < NPART; ++part)
-                        pgr[s][hh][part] = load_uniform(t_row, min(T.tok + 16 * hh + RPP * part, T.w - 1) >> page_shift);
+                        pgr[s][hh][part] = load_uniform(t_row, part_page(min(T.tok + 16 * hh + RPP * part, T.w - 1)));
             }
         } else if constexpr (PATH == kPageLane) {
             // One table read per lane covers the step's pages (at most
@@ -750,15 +771,15 @@ __device__ __forceinline__ void decode_split_body(const pa_decode_params& p, con
             // paths, lookups repeat T's last step once it is exhausted, so
             // that every slot issues the same vector loads.
             const int last  = T.w - 1;
-            const int first = page_shift >= 0 ? T.tok >> page_shift : T.tok / P;   // wave-uniform choice
-            const int lastp = page_shift >= 0 ? last >> page_shift : last / P;
+            const int first = pd.page(T.tok);   // shift or multiply: a wave-uniform choice
+            const int lastp = pd.page(last);
             pent[s] = t_row[min(first + lane, lastp)];
 #pragma unroll
             for (int hh = 0; hh < NH; ++hh)
 #pragma unroll
                 for (int part = 0; part < NPART; ++part) {
                     const int tk = min(T.tok + 16 * hh + RPP * part + lane / CPR, last);
-                    const int qk = page_shift >= 0 ? tk >> page_shift : tk / P;
+                    const int qk = pd.page(tk);
                     plk[s][hh][part] = 4 * (qk - first);
                     psl[s][hh][part] = tk - qk * P;
                 }
@@ -769,13 +790,13 @@ __device__ __forceinline__ void decode_split_body(const pa_decode_params& p, con
 #pragma unroll
             for (int hh = 0; hh < NH; ++hh) {
                 const int tk = min(T.tok + 16 * hh + c, last);
-                const int qk = PATH == kPageQuad ? (tk >> page_shift) : tk / P;
+                const int qk = PATH == kPageQuad ? (tk >> pd.shift) : tk / P;
                 pk[s][hh] = t_row[qk];
                 sk[s][hh] = tk - qk * P;
                 if constexpr (PATH == kPageQuad) {
                     // The lane's 4 V tokens share one page (page_size % 4 == 0).
                     const int tv = min(T.tok + 16 * hh + 4 * kb, last & ~3);
-                    const int qv = tv >> page_shift;
+                    const int qv = tv >> pd.shift;
                     pv[s][hh][0] = t_row[qv];
                     sv[s][hh][0] = tv - qv * P;
                 } else {
@@ -872,7 +893,7 @@ __device__ __forceinline__ void decode_split_body(const pa_decode_params& p, con
                             u32x2, __builtin_amdgcn_raw_buffer_load_b64(vrs, v_lane_off + r * ROW, 0, kAux<NT>));
                 }
             }
-        } else if constexpr (PATH == kPageRuns) {
+        } else if constexpr (RUNS) {
 #pragma unroll
             for (int hh = 0; hh < NH; ++hh)
 #pragma unroll
@@ -882,7 +903,7 @@ __device__ __forceinline__ void decode_split_body(const pa_decode_params& p, con
                     const int nv = __builtin_amdgcn_readfirstlane(l_more ? max(0, min(RPP, L.w - t)) : 0);
                     const size_t row0 =
                         static_cast<size_t>(__builtin_amdgcn_readfirstlane(pgr[s][hh][part])) * page_bytes +
-                        static_cast<uint32_t>((L.h * P + (bt & (P - 1))) * ROW);
+                        static_cast<uint32_t>((L.h * P + part_slot(bt)) * ROW);
                     const __amdgpu_buffer_rsrc_t krs = buffer_rsrc(kbase + row0, nv * ROW);
                     const __amdgpu_buffer_rsrc_t vrs = buffer_rsrc(vbase + row0, nv * ROW);
                     if constexpr (DMA) {
@@ -1273,16 +1294,20 @@ template <int G, int NG, int DEPTH, int PATH>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(PA_FP16_WAVES_PER_EU)))
 void decode_split_kernel_f16(const int32_t* __restrict__ cta, const int32_t* __restrict__ segp,
                              const int32_t* __restrict__ tbl, const int32_t* __restrict__ sid, int num_units,
-                             int page_shift, const int32_t* __restrict__ isb, const pa_decode_params p) {
-    decode_split_body<2, G, NG, DEPTH, PATH>(p, cta, num_units, page_shift, tbl, sid, segp, isb);
+                             int page_shift, const int32_t* __restrict__ isb, uint32_t page_magic,
+                             const pa_decode_params p) {
+    decode_split_body<2, G, NG, DEPTH, PATH>(p, cta, num_units, PageDiv{page_shift, page_magic}, tbl, sid, segp,
+                                              isb);
 }
 
 template <int G, int NG, int DEPTH, int PATH>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(PA_FP8_WAVES_PER_EU)))
 void decode_split_kernel_fp8(const int32_t* __restrict__ cta, const int32_t* __restrict__ segp,
                              const int32_t* __restrict__ tbl, const int32_t* __restrict__ sid, int num_units,
-                             int page_shift, const int32_t* __restrict__ isb, const pa_decode_params p) {
-    decode_split_body<1, G, NG, DEPTH, PATH>(p, cta, num_units, page_shift, tbl, sid, segp, isb);
+                             int page_shift, const int32_t* __restrict__ isb, uint32_t page_magic,
+                             const pa_decode_params p) {
+    decode_split_body<1, G, NG, DEPTH, PATH>(p, cta, num_units, PageDiv{page_shift, page_magic}, tbl, sid, segp,
+                                              isb);
 }
 
 // ---------------------------------------------------------------------------
@@ -1423,42 +1448,64 @@ template <int EB> constexpr int kPow2Depth = kLdsDma && Tune<EB>::stage ? 1 : Tu
 template <int EB> constexpr int kRunsDepth = kLdsDma ? 1 : Tune<EB>::depth;
 
 template <int EB, int G, int NG, int DEPTH, int PATH>
-hipError_t launch_split_p(const pa_decode_params& p, int shift, hipStream_t s) {
+hipError_t launch_split_p(const pa_decode_params& p, const PageDiv& pd, hipStream_t s) {
     const int blocks = (p.num_ctas + kWaves - 1) / kWaves;
     if constexpr (EB == 2)
         hipLaunchKernelGGL((decode_split_kernel_f16<G, NG, DEPTH, PATH>), dim3(blocks), dim3(64 * kWaves), 0, s,
-                           p.cta_seg_begin, p.segments, p.block_table, p.slot_ids, p.num_ctas, shift,
-                           p.item_seg_begin, p);
+                           p.cta_seg_begin, p.segments, p.block_table, p.slot_ids, p.num_ctas, pd.shift,
+                           p.item_seg_begin, pd.magic, p);
     else
         hipLaunchKernelGGL((decode_split_kernel_fp8<G, NG, DEPTH, PATH>), dim3(blocks), dim3(64 * kWaves), 0, s,
-                           p.cta_seg_begin, p.segments, p.block_table, p.slot_ids, p.num_ctas, shift,
-                           p.item_seg_begin, p);
+                           p.cta_seg_begin, p.segments, p.block_table, p.slot_ids, p.num_ctas, pd.shift,
+                           p.item_seg_begin, pd.magic, p);
     return hipGetLastError();
+}
+
+PageDiv page_div(int page_size) {
+    const uint32_t P = static_cast<uint32_t>(page_size);
+    if ((P & (P - 1)) == 0) return {__builtin_ctz(P), 0u};
+    const int l = 32 - __builtin_clz(P - 1);   // ceil(log2 P), at least 2
+    return {~(l - 1), static_cast<uint32_t>((1ull << (31 + l)) / P + 1)};
 }
 
 template <int EB, int G>
 hipError_t launch_split_g(const pa_decode_params& p, hipStream_t s) {
-    const int  P     = p.page_size;
-    const bool pow2  = (P & (P - 1)) == 0;
-    const int  shift = pow2 ? __builtin_ctz(static_cast<unsigned>(P)) : 0;
+    const int     P     = p.page_size;
+    const PageDiv pd    = page_div(P);
+    const bool    pow2  = pd.shift >= 0;
+    // Byte offsets of one page and of one (kv head, slot) inside it are 32-bit
+    // on the paths that look a page up once per half or part.
+    const bool    small = static_cast<long long>(p.num_kv_heads) * P * kRowBytes<EB> < (1ll << 31);
+    auto need_small = [&] {
+        if (!small) throw std::invalid_argument("decode: page_size * num_kv_heads * row bytes must be below 2^31");
+    };
     if (pow2 && P >= 16) {
-        // Byte offsets of one page and of one (kv head, slot) inside it are 32-bit.
-        if (static_cast<long long>(p.num_kv_heads) * P * kRowBytes<EB> >= (1ll << 31))
-            throw std::invalid_argument("decode: page_size * num_kv_heads * row bytes must be below 2^31");
-        return launch_split_p<EB, G, Tune<EB>::step, kPow2Depth<EB>, kPagePow2>(p, shift, s);
+        need_small();
+        return launch_split_p<EB, G, Tune<EB>::step, kPow2Depth<EB>, kPagePow2>(p, pd, s);
     }
     if constexpr (EB == 2 || Tune<EB>::stage) {
         // Pages of whole 1 KiB parts (4 fp16 rows, 8 FP8 rows) through the LDS stage.
+        constexpr int RPP = 1024 / kRowBytes<EB>;
         if (P == 8 || (EB == 2 && P == 4)) {
-            if (static_cast<long long>(p.num_kv_heads) * P * kRowBytes<EB> >= (1ll << 31))
-                throw std::invalid_argument("decode: page_size * num_kv_heads * row bytes must be below 2^31");
-            return launch_split_p<EB, G, Tune<EB>::step, kRunsDepth<EB>, kPageRuns>(p, shift, s);
+            need_small();
+            return launch_split_p<EB, G, Tune<EB>::step, kRunsDepth<EB>, kPageRuns>(p, pd, s);
         }
-        // Any other size: per-lane rows through the LDS stage (shift -1: divide).
-        return launch_split_p<EB, G, Tune<EB>::step, kLaneDepth<EB>, kPageLane>(p, pow2 ? shift : -1, s);
+        // The same for pages that are no powers of two but hold whole parts
+        // (pages past the 32-bit offsets stay on the per-lane path): one scalar
+        // table read and buffer resource per part instead of a vector table
+        // read, four lane exchanges and 64-bit lane addresses per step. Same
+        // box, us per step, per-lane path -> this one: 37 ragged FP8 rows of up
+        // to 3001 tokens, 64 query heads, 24-token pages 23.8 -> 22.4; 32 x
+        // 8192 fp16 and 64 x 8192 FP8, 24-token pages 161.0 -> 159.3 and 163.3
+        // -> 160.3. Sizes below one part (fp16 1 to 3, FP8 1 to 7) and sizes
+        // whose pages cut a part in two have no such resource.
+        if (!pow2 && P % RPP == 0 && small)
+            return launch_split_p<EB, G, Tune<EB>::step, kRunsDepth<EB>, kPageRunsDiv>(p, pd, s);
+        // Any other size: per-lane rows through the LDS stage.
+        return launch_split_p<EB, G, Tune<EB>::step, kLaneDepth<EB>, kPageLane>(p, pd, s);
     } else {
-        if (pow2 && P >= 4) return launch_split_p<EB, G, Tune<EB>::step, kLaneDepth<EB>, kPageQuad>(p, shift, s);
-        return launch_split_p<EB, G, Tune<EB>::step, kLaneDepth<EB>, kPageAny>(p, shift, s);
+        if (pow2 && P >= 4) return launch_split_p<EB, G, Tune<EB>::step, kLaneDepth<EB>, kPageQuad>(p, pd, s);
+        return launch_split_p<EB, G, Tune<EB>::step, kLaneDepth<EB>, kPageAny>(p, pd, s);
     }
 }
 
