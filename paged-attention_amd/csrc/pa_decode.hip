@@ -61,10 +61,11 @@
 //     8192 tokens over 2048 units) is then complete; a row that spans blocks
 //     (up to 8) leaves one device-coherent partial per block, and the last
 //     of its blocks to arrive (a per-row counter) combines them, in block
-//     order. No merge launch is needed. Otherwise (rows over more blocks, or
-//     caller plans that do not keep a row's segments in consecutive units)
-//     every split segment's partial goes to the plan's workspace for the
-//     merge kernel.
+//     order. No merge launch is needed. Where a row spans more blocks
+//     (block_merge 3) each block leaves such a partial for the merge kernel.
+//     Otherwise (caller plans that do not keep a row's segments in consecutive
+//     units, and rows of one query head over fewer than 64 blocks) every split
+//     segment's partial goes to the plan's workspace for the merge kernel.
 
 #include "pa_device.hpp"
 
@@ -479,12 +480,13 @@ __device__ __forceinline__ void combine_blocks(const pa_decode_params& p, const 
 // slower where a block holds one or two runs and no faster elsewhere.
 //
 // An item whose segments all lie in this block (block_merge 1: every split
-// item) is written as fp16. With block_merge 2 an item may also span blocks
+// item) is written as fp16. With block_merge 2 and 3 an item may also span blocks
 // (its k-th segment runs in unit u0 + k, so it continues from the previous
 // block at the block's first slot and into the next at its last): the block's
 // average becomes one partial row of the item, at the workspace slot of the
 // item's first segment in the block, with LSE max + log2(sum of weights).
-// After every thread's stores are complete, one lane per such item adds one to
+// Under block_merge 3 the merge kernel does the rest. Under 2,
+// after every thread's stores are complete, one lane per such item adds one to
 // the item's counter; the block that brings it to the item's block count
 // resets it to zero and combines the item's block partials, in block order, as
 // the merge kernel does (so the result does not depend on which block is
@@ -499,7 +501,7 @@ __device__ __forceinline__ void block_merge(const pa_decode_params& p, const Slo
     static_assert(NS == 16, "the slots fit the low lanes of a wave");
     const int  lane  = tid & 63;
     const int  wave  = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const bool chain = p.block_merge == 2;
+    const bool chain = p.block_merge >= 2;
     if (tid == 0) stamp(16);
     const Slot     mine   = slots[lane & (NS - 1)];   // lane j holds slot j
     const uint32_t filled = static_cast<uint32_t>(__builtin_amdgcn_ballot_w64(lane < NS && mine.item >= 0));
@@ -582,7 +584,7 @@ __device__ __forceinline__ void block_merge(const pa_decode_params& p, const Slo
             }
         }
     }
-    if (!chain) return;
+    if (p.block_merge != 2) return;   // 3: the merge kernel combines the block partials
     // Items of this block that span blocks: its first run, its last, or both
     // (sa; sb when there are two).
     auto span_of = [&](uint32_t from) {
@@ -1321,13 +1323,20 @@ void decode_split_kernel_fp8(const int32_t* __restrict__ cta, const int32_t* __r
 // lane (no separate pass for the maximum: one dependent round trip fewer);
 // lanes of the same dims combine by shuffles, waves in LDS.
 //
+// With unit0 (block_merge 3) the partials are those the blocks left, an eighth
+// as many: the split kernel leaves an eighth of the dirty lines to write back
+// before this kernel may start, and this one reads an eighth (us per step: one
+// row of 131072, one kv head 20.8 -> 16.1; 1 x 4096 fp16 10.0 -> 8.9).
+//
 // The arrays it reads first come ahead of the params struct, preloaded in SGPRs
 // (as for the split kernels).
 template <int G, int WAVES, int DS>
 __global__ __launch_bounds__(64 * WAVES) void decode_merge_kernel(const int32_t* __restrict__ isb,
                                                                   const float* __restrict__ part_out,
                                                                   const float* __restrict__ part_lse,
-                                                                  int num_kv_heads, const pa_decode_params p) {
+                                                                  int num_kv_heads,
+                                                                  const int32_t* __restrict__ unit0,
+                                                                  const pa_decode_params p) {
     constexpr int LPS = DS / 4;      // lanes per segment
     constexpr int SPW = 64 / LPS;    // segments per wave per pass
     // The combine below exchanges lanes 4, 8, 16 and 32 apart only.
@@ -1338,7 +1347,12 @@ __global__ __launch_bounds__(64 * WAVES) void decode_merge_kernel(const int32_t*
     const int item = b * num_kv_heads + hqi / G;
     const int g    = hqi % G;
     const int s0 = isb[item];
-    const int n  = isb[item + 1] - s0;
+    int n  = isb[item + 1] - s0;
+    // Block partials (unit0 given): the item's j-th partial sits at its first
+    // segment in the j-th block it spans; an item inside one block is done.
+    const int u0 = unit0 ? unit0[item] : 0;
+    const int j0 = u0 / kWaves;
+    if (unit0) n = (u0 + n - 1) / kWaves - j0 + 1;
     if (n <= 1) return;
 
     __shared__ float4 acc_lds[WAVES][LPS];
@@ -1357,7 +1371,7 @@ __global__ __launch_bounds__(64 * WAVES) void decode_merge_kernel(const int32_t*
     float  den = 0.f, m = -INFINITY;
 #pragma unroll 4
     for (int i = wave * SPW + sl; i < n; i += WAVES * SPW) {
-        const size_t sg  = static_cast<size_t>(s0 + i);
+        const size_t sg  = static_cast<size_t>(s0 + (unit0 ? max(0, kWaves * (j0 + i) - u0) : i));
         const float  lse = part_lse[sg * G + g];
         const float4 o   = *reinterpret_cast<const float4*>(part_out + (sg * G + g) * kHeadDim + d0 + 4 * dq);
         const float  mn  = fmaxf(m, lse);
@@ -1527,13 +1541,15 @@ template <int G, int DS>
 hipError_t launch_merge_gd(const pa_decode_params& p, hipStream_t s) {
     const dim3 grid(p.num_q_heads, p.batch, kHeadDim / DS);
     constexpr int SPW = 256 / DS;    // segments one wave covers per pass
-    const int m = p.max_item_segments;
+    const bool blocks = p.block_merge == 3;
+    const int  m      = blocks ? (p.max_item_segments + kWaves - 1) / kWaves + 1 : p.max_item_segments;
+    const int32_t* unit0 = blocks ? p.merge_counters + plan_item_units(p.batch * p.num_kv_heads) : nullptr;
     if (m > 0 && m <= 4 * SPW)
         hipLaunchKernelGGL((decode_merge_kernel<G, 1, DS>), grid, dim3(64), 0, s, p.item_seg_begin, p.partial_out,
-                           p.partial_lse, p.num_kv_heads, p);
+                           p.partial_lse, p.num_kv_heads, unit0, p);
     else
         hipLaunchKernelGGL((decode_merge_kernel<G, 4, DS>), grid, dim3(256), 0, s, p.item_seg_begin, p.partial_out,
-                           p.partial_lse, p.num_kv_heads, p);
+                           p.partial_lse, p.num_kv_heads, unit0, p);
     return hipGetLastError();
 }
 
@@ -1600,11 +1616,12 @@ int kernel_units_per_cu(int dtype, int group) {
 }
 
 // A plan's split rows are merged either by the merge kernel (needs_merge) or
-// inside the split kernel (block_merge), never both: with block_merge the
-// workspace holds partial rows only at the slots the split kernel merges
-// through, and the merge kernel would read the others unwritten.
+// inside the split kernel (block_merge 1 and 2), never both: the workspace then
+// holds partial rows only at the slots the split kernel merges through, and the
+// merge kernel would read the others unwritten. (Under block_merge 3 it reads
+// those slots only.)
 void check_merge_fields(const pa_decode_params& p) {
-    if (p.needs_merge && p.block_merge)
+    if (p.needs_merge && p.block_merge && p.block_merge != 3)
         throw std::invalid_argument("decode: needs_merge and block_merge exclude each other (bind sets them)");
 }
 
@@ -1620,9 +1637,9 @@ hipError_t launch_decode_split(int dtype, const pa_decode_params& p, hipStream_t
         throw std::invalid_argument("decode: null pointer in params");
     if ((p.needs_merge || p.block_merge) && (!p.partial_out || !p.partial_lse))
         throw std::invalid_argument("decode: split rows need the partial workspace");
-    if (p.block_merge < 0 || p.block_merge > 2) throw std::invalid_argument("decode: block_merge must be 0, 1 or 2");
-    if (p.block_merge == 2 && !p.merge_counters)
-        throw std::invalid_argument("decode: block_merge 2 needs the plan's merge counters");
+    if (p.block_merge < 0 || p.block_merge > 3) throw std::invalid_argument("decode: block_merge must be 0, 1, 2 or 3");
+    if (p.block_merge >= 2 && !p.merge_counters)
+        throw std::invalid_argument("decode: block_merge 2 and 3 need the plan's merge counters");
     return dtype == PA_KV_FP16 ? launch_split_e<2>(p, g, s) : launch_split_e<1>(p, g, s);
 }
 
@@ -1631,7 +1648,8 @@ hipError_t launch_decode_merge(int dtype, const pa_decode_params& p, hipStream_t
     const int g = checked_group(p);
     check_merge_fields(p);
     if (!p.needs_merge || p.batch <= 0) return hipSuccess;
-    if (!p.partial_out || !p.partial_lse || !p.item_seg_begin || !p.out)
+    if (!p.partial_out || !p.partial_lse || !p.item_seg_begin || !p.out ||
+        (p.block_merge == 3 && !p.merge_counters))
         throw std::invalid_argument("decode merge: null pointer in params");
     switch (g) {
         case 1: return launch_merge_g<1>(p, s);

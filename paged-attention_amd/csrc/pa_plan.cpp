@@ -105,46 +105,68 @@ void check_dtype(int dtype) {
     if (dtype != PA_KV_FP16 && dtype != PA_KV_FP8_E4M3)
         throw std::invalid_argument("unknown kv dtype " + std::to_string(dtype));
 }
-constexpr int kChainMaxBlocks = 8;    // blocks one item may span under block_merge 2
-int plan_merge_mode(const pa_plan& plan) {
+// How a plan's split items lie in units and blocks.
+struct SplitShape {
+    bool split       = false;   // some item has several segments
+    bool slots       = true;    // every split segment is its unit's first or last
+    bool in_block    = true;    // no item spans blocks
+    bool consecutive = true;    // an item's k-th segment runs in unit u0 + k
+    int  max_blocks  = 0;       // most blocks of one split item
+};
+SplitShape split_shape(const pa_plan& plan, std::vector<int32_t>* item_unit) {
+    SplitShape sh;
     const size_t nseg = plan.segments.size() / 4;
-    if (nseg <= static_cast<size_t>(plan.items)) return 0;   // no split items
-    // The split kernel keeps a unit's split segments in two LDS slots: they
-    // must be the unit's first and last segments (true of every make_plan cut).
+    sh.split = nseg > static_cast<size_t>(plan.items);
+    if (!sh.split) return sh;
     std::vector<int32_t> unit_of(nseg, 0);
     for (int u = 0; u < plan.num_ctas; ++u)
         for (int sg = plan.cta_seg_begin[u]; sg < plan.cta_seg_begin[u + 1]; ++sg)
             unit_of[static_cast<size_t>(sg)] = u;
-    bool in_block = true, consecutive = true;
+    if (item_unit) item_unit->resize(static_cast<size_t>(plan.items));
     for (int i = 0; i < plan.items; ++i) {
         const int a = plan.item_seg_begin[i], z = plan.item_seg_begin[i + 1];
-        if (z - a <= 1) continue;
         const int u0 = unit_of[static_cast<size_t>(a)];
+        if (item_unit) (*item_unit)[static_cast<size_t>(i)] = u0;
+        if (z - a <= 1) continue;
         const int nb = unit_of[static_cast<size_t>(z - 1)] / pa::kBlockUnits - u0 / pa::kBlockUnits + 1;
-        if (nb > 1) in_block = false;
-        // The split kernel's combine of a spanning item runs on one CU and
-        // reads one partial per block: past 8 blocks per item the merge
-        // kernel, which spreads every item over many CUs, is as fast or
-        // faster (one MI355X: at 16 blocks per item 0.4-1.3 us faster in the
-        // split kernel back to back but 0.9-1.6 us slower after a cache
-        // flush, and slower either way on half-filled grids; at 32 blocks
-        // 0.5-2.7 us slower). It addresses the partial rows with 32-bit
-        // offsets (segments x 8 heads x 128 floats).
-        if (nb > kChainMaxBlocks || z - a >= (1 << 19)) consecutive = false;
+        sh.max_blocks = std::max(sh.max_blocks, nb);
+        if (nb > 1) sh.in_block = false;
+        if (z - a >= (1 << 19)) sh.consecutive = false;   // 32-bit offsets of 8 heads x 128 floats
         for (int sg = a; sg < z; ++sg) {
             const int u = unit_of[static_cast<size_t>(sg)];
-            if (sg != plan.cta_seg_begin[u] && sg != plan.cta_seg_begin[u + 1] - 1) return 0;
-            if (u != u0 + (sg - a)) consecutive = false;
+            if (sg != plan.cta_seg_begin[u] && sg != plan.cta_seg_begin[u + 1] - 1) sh.slots = false;
+            if (u != u0 + (sg - a)) sh.consecutive = false;
         }
     }
-    if (in_block) return 1;
-    // Chained merge: a block finds an item's other blocks from the unit of the
-    // item's first segment, which needs the item's k-th segment in unit u0 + k.
+    return sh;
+}
+// The split kernel's combine of a spanning item runs on one CU and reads one
+// partial per block. Up to 8 blocks per item that is as fast as a merge launch
+// or faster; past 8 the split kernel leaves one partial per block and the merge
+// kernel, which spreads every item over many CUs, combines those (one MI355X,
+// us per step, combine in the split kernel against this: 16 blocks per item,
+// 2 x 2048 fp16 9.9 / 8.7, 2 x 16384 FP8 16.9 / 16.2; 32 blocks, 1 x 131072 FP8
+// 47.4 / 45.8, 1 x 16384 fp16 19.0 / 15.7).
+constexpr int kChainMaxBlocks = 8;
+// One query head per kv head leaves partials of 512 bytes per segment: merging
+// them per block first costs what it saves (1 x 131072 FP8 44.6 without, 45.2
+// with; 1 x 16384 fp16 14.7 / 15.1; 2 x 16384 FP8 level) until an item has
+// hundreds of segments (one kv head, 1 x 131072 fp16, 256 blocks: 18.2 / 15.6).
+constexpr int kOneHeadMinBlocks = 64;
+int merge_mode_of(const SplitShape& sh, int max_blocks) {
+    // The split kernel keeps a unit's split segments in two LDS slots: they
+    // must be the unit's first and last segments (true of every make_plan cut).
+    if (!sh.split || !sh.slots) return 0;
+    if (sh.in_block) return 1;
+    // Merged across blocks: a block finds an item's other blocks from the unit
+    // of the item's first segment, which needs the item's k-th segment in unit
+    // u0 + k.
 #if PA_CHAIN_MERGE
-    if (consecutive) return 2;
+    if (sh.consecutive && sh.max_blocks <= max_blocks) return 2;
 #endif
     return 0;
 }
+int plan_merge_mode(const pa_plan& plan) { return merge_mode_of(split_shape(plan, nullptr), kChainMaxBlocks); }
 void make_plan_impl(pa_plan& plan, int dtype, const int32_t* lens, int batch, int hq, int hkv, int hd,
                     int num_ctas) {
     const int group = group_of(hq, hkv);
@@ -217,7 +239,18 @@ void device_plan_upload(pa_device_plan& dp, const pa_plan& plan, int group, int 
     const size_t o_item  = o_cta + round4(plan.cta_seg_begin.size());
     const size_t o_extra = o_item + round4(plan.item_seg_begin.size());
     const size_t o_ctr   = o_extra + round4(n_extra);   // per-item merge counters, uploaded as zeros
-    const size_t total   = o_ctr + round4(static_cast<size_t>(plan.items));
+    std::vector<int32_t> item_unit;
+    const SplitShape shape = split_shape(plan, &item_unit);
+    const int  in_kernel = merge_mode_of(shape, kChainMaxBlocks);
+    // Past kChainMaxBlocks: block partials for the merge kernel (block_merge 3),
+    // where the split kernel can find an item's part of a block. Same box, us per
+    // step, every segment's partial / block partials: one row of 131072, one kv
+    // head 20.8 / 16.1; 1 x 4096 fp16 10.0 / 8.9; 2 x 2048, 64 query heads 12.0 /
+    // 9.4; 3 ragged rows to 30000 21.9 / 20.5; 1 x 131072 FP8 46.4 / 45.9.
+    const bool blocks    = in_kernel == 0 && merge_mode_of(shape, INT_MAX) == 2 &&
+                        (group > 1 || shape.max_blocks >= kOneHeadMinBlocks);
+    const size_t o_unit  = o_ctr + pa::plan_item_units(plan.items);
+    const size_t total   = blocks ? o_unit + round4(item_unit.size()) : o_unit;
     if (total > dp.ints_cap) {
         // Growing frees the old block, which decodes queued before may still
         // read: wait for them first (growth only happens for a plan larger
@@ -235,7 +268,8 @@ void device_plan_upload(pa_device_plan& dp, const pa_plan& plan, int group, int 
     std::copy(plan.cta_seg_begin.begin(), plan.cta_seg_begin.end(), st.host + o_cta);
     std::copy(plan.item_seg_begin.begin(), plan.item_seg_begin.end(), st.host + o_item);
     if (n_extra) std::copy(extra, extra + n_extra, st.host + o_extra);
-    std::fill(st.host + o_ctr, st.host + total, 0);
+    std::fill(st.host + o_ctr, st.host + o_unit, 0);
+    if (blocks) std::copy(item_unit.begin(), item_unit.end(), st.host + o_unit);
     pa::hip_check(hipMemcpyAsync(dp.ints, st.host, total * sizeof(int32_t), hipMemcpyHostToDevice, s),
                   "hipMemcpyAsync plan");
     release_stage(st, s);
@@ -256,8 +290,8 @@ void device_plan_upload(pa_device_plan& dp, const pa_plan& plan, int group, int 
     dp.partial_lse = dp.partial_out ? dp.partial_out + rows * head_dim : nullptr;
     dp.num_ctas = plan.num_ctas;
     dp.num_segments = static_cast<int>(nseg);
-    dp.block_merge = plan_merge_mode(plan);
-    dp.needs_merge = dp.block_merge == 0 && nseg > static_cast<size_t>(plan.items) ? 1 : 0;
+    dp.block_merge = blocks ? 3 : in_kernel;
+    dp.needs_merge = blocks || (in_kernel == 0 && shape.split) ? 1 : 0;
     dp.max_item_segments = 0;
     for (int i = 0; i < plan.items; ++i)
         dp.max_item_segments = std::max(dp.max_item_segments, plan.item_seg_begin[i + 1] - plan.item_seg_begin[i]);

@@ -86,7 +86,7 @@ pa_status pa_decode_static(int dtype, const pa_decode_params* p, int num_segment
                                         ") differs from the bound plan's (" + std::to_string(p->num_segments) + ")");
         const long items      = static_cast<long>(p->batch) * p->num_kv_heads;
         const bool split_rows = p->num_segments > items;
-        if (split_rows && !p->block_merge && !p->needs_merge)
+        if (split_rows && (!p->block_merge || p->block_merge == 3) && !p->needs_merge)
             throw std::invalid_argument("decode_static: a plan with split rows needs needs_merge or block_merge");
         const size_t group = static_cast<size_t>(p->num_q_heads / p->num_kv_heads);
         const size_t rows  = static_cast<size_t>(p->num_segments) * group;

@@ -132,9 +132,9 @@ class DecodePlan:
 
     @property
     def merge_mode(self) -> int:
-        """pa_decode_params.block_merge that DevicePlan.bind sets for this plan:
-        0 (merge kernel), 1 (split items merged inside one block), 2 (items
-        spanning blocks merged by the split kernel too)."""
+        """How the plan's split items are merged: 0 (merge kernel; bind may have
+        the blocks merge their own parts first), 1 (split items merged inside
+        one block), 2 (items spanning blocks merged by the split kernel too)."""
         if self.handle is None:
             raise ValueError("plan has no native handle")
         out = ctypes.c_int(0)

@@ -34,7 +34,7 @@ def _check(fp8, lens, group, hkv, handle, mode, page=16, repeats=6):
         p.batch, p.num_q_heads, p.num_kv_heads, p.head_dim, p.page_size = len(lens), hq, hkv, D, page
         p.sm_scale, p.k_scale, p.v_scale = pa_amd.sm_scale(D), ks, vs
         dplan.bind(p)
-        assert p.block_merge == mode and p.needs_merge == 0
+        assert p.block_merge == mode and p.needs_merge == (mode == 3)
         if rep == repeats:
             p.block_merge, p.needs_merge = 0, 1   # the merge kernel on the same plan
         pa_amd.paged_decode(dt, p)
@@ -90,3 +90,21 @@ def test_run_of_sixteen_slots(group):
         _check(False, [256, 29], group, 1, h.value, 1)
     finally:
         pa_amd._lib.load().pa_plan_destroy(h.value)
+
+
+@pytest.mark.parametrize("lens,ctas,group,hkv", [
+    ([4096], 0, 4, 8),                          # one tile per unit, 32 blocks per row
+    ([131072], 0, 1, 1),                        # one query head, 256 blocks
+    ([131072 - 7], 0, 8, 1),
+    ([30000, 17, 1, 1100, 9000], 0, 2, 8),      # rows inside a block, over a few, over many
+    ([2048, 2048], 0, 8, 8),                    # 16 blocks
+    ([700, 5000], 700, 4, 2),
+], ids=["one_tile", "one_head", "g8", "ragged", "two_rows", "few_units"])
+@pytest.mark.parametrize("fp8", [False, True], ids=["fp16", "fp8"])
+def test_block_partials_for_the_merge_kernel(fp8, lens, ctas, group, hkv):
+    """Rows over more than 8 blocks: the blocks merge their own part first."""
+    if fp8:
+        lens = [2 * n for n in lens]            # the tile is twice as long: the same units
+    plan = _plan(fp8, lens, group, hkv, ctas)
+    assert plan.merge_mode == 0
+    _check(fp8, lens, group, hkv, plan.handle.value, 3, repeats=3)
