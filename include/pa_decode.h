@@ -161,7 +161,7 @@ void      pa_device_plan_destroy(pa_device_plan* dp);
 /* decode.cu:131-146 DevicePlan::upload: grow-only device copies of the plan plus
  * the partial workspace (segments * group * (head_dim + 1) floats). Rejects a
  * plan whose segments do not start on multiples of 16 tokens. The plan's arrays
- * go through pinned staging as one copy queued on `stream`; the call does not
+ * go through pinned staging, read by one copy kernel queued on `stream`; the call does not
  * synchronize the stream (it waits only when 8 of its uploads are still in
  * flight, and synchronizes once when a plan outgrows every earlier one), and
  * the host plan may change or go as soon as it returns. Decodes queued earlier
@@ -324,11 +324,12 @@ pa_status pa_cache_append(pa_cache* cache, int slot, const uint16_t* d_k, const 
  * tokens to slots[i] for i = 0..n-1 (host arrays; a slot may repeat, its
  * tokens then follow in order). d_k / d_v hold every token, concatenated in
  * entry order: [sum(counts)][Hkv][D] fp16. Pages are reserved all-or-nothing
- * (*appended = 0 and nothing changed when the pool lacks pages). The new
- * block-table entries and lengths go over in one pinned host-to-device copy and
- * one kernel writes them together with every token (copy or E4M3 quantize): two
- * stream operations, no stream synchronization. The call returns once its host
- * staging is queued; it waits only when 8 of its batches are still in flight. */
+ * (*appended = 0 and nothing changed when the pool lacks pages). One kernel
+ * writes the new block-table entries and lengths together with every token
+ * (copy or E4M3 quantize), no stream synchronization: they travel in its
+ * arguments, or, past about 3.5 KB (some 290 new pages), through pinned staging
+ * and a copy kernel before it. Then the call waits only when 8 such batches are
+ * still in flight. */
 pa_status pa_cache_append_batch(pa_cache* cache, const int32_t* slots, const int32_t* counts, int n,
                                 const uint16_t* d_k, const uint16_t* d_v, void* stream, int* appended);
 pa_status pa_cache_release(pa_cache* cache, int slot);

@@ -1,8 +1,9 @@
 // gfx950 kernels around the decode path:
 //
 //   append_kernel        fp16 copy / FP8 E4M3 quantize + page scatter (paged_kv_cache.cu:15-39)
-//   append_batch_kernel  the same for a whole decode step's appends across sequences, plus the
-//                        new block-table entries and lengths, in one launch
+//   append_batch_kernel, append_inline_kernel  the same for a whole decode step's appends across
+//                        sequences, plus the new block-table entries and lengths, in one launch
+//   stage_copy_kernel    pinned host memory to the device (plans, long appends' metadata)
 //   gather_kernel        block-table resolution probe (the decode kernel's row address function)
 //   stream_read_kernel   streaming read: cache flush and plain-copy ceiling (bench_decode.cu:70-78)
 //   stream_read_chunked_kernel  the same read with one contiguous span per wave (best read rate)
@@ -15,6 +16,7 @@
 #include <algorithm>
 #include <climits>
 #include <cmath>
+#include <cstddef>
 #include <cstdint>
 #include <stdexcept>
 #include <string>
@@ -183,14 +185,23 @@ __global__ __launch_bounds__(256) void append_kernel(const uint16_t* __restrict_
     store_chunk<EB>(in, k_cache, v_cache, dst, inv_k, inv_v);
 }
 
+// An append whose meta travels in the kernel's arguments (N ints): no staging
+// buffer, no copy before the kernel. A decode step's tokens of up to 128
+// sequences fit, and prompts of some 290 new pages.
+template <int N>
+struct AppendInline {
+    AppendBatch a;
+    alignas(16) int32_t meta[N];
+};
+
 // The chunk of thread idx of append_batch_kernel.
 template <int EB>
-__device__ __forceinline__ void append_batch_chunk(const AppendBatch& a, int idx) {
+__device__ __forceinline__ void append_batch_chunk(const AppendBatch& a, const int32_t* meta, int idx) {
     constexpr int DIMS = kAppendDims<EB>, CPR = kHeadDim / DIMS;
-    const int32_t* tok_begin = a.meta;
-    const int32_t* old_len   = a.meta + a.n_ent;
-    const int32_t* pl_begin  = a.meta + 2 * a.n_ent;
-    const int32_t* pages     = a.meta + 3 * a.n_ent;
+    const int32_t* tok_begin = meta;
+    const int32_t* old_len   = meta + a.n_ent;
+    const int32_t* pl_begin  = meta + 2 * a.n_ent;
+    const int32_t* pages     = meta + 3 * a.n_ent;
     const int chunk = static_cast<unsigned>(idx) % CPR;
     const int th    = static_cast<unsigned>(idx) / CPR;
     const int h     = th % a.hkv;
@@ -228,10 +239,10 @@ __device__ __forceinline__ void append_batch_chunk(const AppendBatch& a, int idx
 // its page in the entry's page list: table entries are read from the staging
 // copy, never from the block table this launch is writing.
 template <int EB>
-__global__ __launch_bounds__(256) void append_batch_kernel(const AppendBatch a) {
+__device__ __forceinline__ void append_batch_body(const AppendBatch& a, const int32_t* meta) {
     constexpr int CPR = kHeadDim / kAppendDims<EB>;
     const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    const int32_t* tab       = a.meta + 3 * a.n_ent + a.n_pl;
+    const int32_t* tab       = meta + 3 * a.n_ent + a.n_pl;
     const int32_t* lens      = tab + 2 * a.n_tab;
     // A thread's table entry and length are read first and written last, so
     // that every load of the thread is issued before its first store. Both
@@ -242,9 +253,34 @@ __global__ __launch_bounds__(256) void append_batch_kernel(const AppendBatch a) 
         u32x2, __builtin_amdgcn_raw_buffer_load_b64(buffer_rsrc(tab, 8 * a.n_tab), 8 * min(idx, a.n_tab), 0, 0));
     const u32x2 lenv = __builtin_bit_cast(
         u32x2, __builtin_amdgcn_raw_buffer_load_b64(buffer_rsrc(lens, 8 * a.n_len), 8 * min(idx, a.n_len), 0, 0));
-    if (idx < a.n_tok * a.hkv * CPR) append_batch_chunk<EB>(a, idx);
+    if (idx < a.n_tok * a.hkv * CPR) append_batch_chunk<EB>(a, meta, idx);
     if (idx < a.n_tab) a.table[tabv[0]] = static_cast<int32_t>(tabv[1]);
     if (idx < a.n_len) a.seq_lens[lenv[0]] = static_cast<int32_t>(lenv[1]);
+}
+
+template <int EB>
+__global__ __launch_bounds__(256) void append_batch_kernel(const AppendBatch a) {
+    append_batch_body<EB>(a, a.meta);
+}
+
+// The meta is read where the arguments lie (the kernel argument segment, which
+// starts with the one argument): indexing a by-value array would copy it to
+// scratch first.
+template <int EB, int N>
+__global__ __launch_bounds__(256) void append_inline_kernel(const AppendInline<N> x) {
+    const uintptr_t args = (uintptr_t)__builtin_amdgcn_kernarg_segment_ptr();
+    append_batch_body<EB>(x.a, reinterpret_cast<const int32_t*>(args + offsetof(AppendInline<N>, meta)));
+}
+
+// Pinned host memory to the device, 16 bytes per thread. Bound by the bus and
+// its latency (56 KB of a 2048-unit plan: 4.0 us). The runtime's copy took 6.3
+// us on a DMA engine plus the decode's wait for another queue, and a new
+// request's host step more than a launch: with this and the arguments' meta
+// above, a step of 30 resident and 2 joining sequences 94.6 -> 85.0 us, of 16
+// and 1 (one-sequence append) 71.9 -> 60.4.
+__global__ __launch_bounds__(256) void stage_copy_kernel(const u32x4* __restrict__ host, u32x4* __restrict__ dev, int n) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) dev[i] = host[i];
 }
 
 // One thread per (token, 8-dim chunk) of one kv head: raw cache bytes out,
@@ -353,16 +389,36 @@ hipError_t launch_append(int dtype, const uint16_t* k, const uint16_t* v, void* 
     return hipGetLastError();
 }
 
-hipError_t launch_append_batch(int dtype, const AppendBatch& a, hipStream_t s) {
+namespace {
+template <int N>
+void launch_append_inline(int dtype, const AppendBatch& a, const int32_t* meta, size_t n, int blocks, hipStream_t s) {
+    AppendInline<N> x;
+    x.a = a;
+    std::copy(meta, meta + n, x.meta);
+    if (dtype == PA_KV_FP16) hipLaunchKernelGGL((append_inline_kernel<2, N>), dim3(blocks), dim3(256), 0, s, x);
+    else hipLaunchKernelGGL((append_inline_kernel<1, N>), dim3(blocks), dim3(256), 0, s, x);
+}
+}  // namespace
+
+hipError_t launch_append_batch(int dtype, const AppendBatch& a, const int32_t* meta, size_t n_meta, hipStream_t s) {
     check_kv_dtype(dtype);
     const int  cpr     = kHeadDim / (dtype == PA_KV_FP16 ? kAppendDims<2> : kAppendDims<1>);
     const long threads = std::max<long>(static_cast<long>(a.n_tok) * a.hkv * cpr, std::max(a.n_tab, a.n_len));
     if (threads <= 0) return hipSuccess;
     const int blocks = static_cast<int>((threads + 255) / 256);
-    if (dtype == PA_KV_FP16)
-        hipLaunchKernelGGL(append_batch_kernel<2>, dim3(blocks), dim3(256), 0, s, a);
-    else
-        hipLaunchKernelGGL(append_batch_kernel<1>, dim3(blocks), dim3(256), 0, s, a);
+    // Two sizes of argument block: the launch writes all of it over the bus.
+    if (meta && n_meta <= 256) launch_append_inline<256>(dtype, a, meta, n_meta, blocks, s);
+    else if (meta) launch_append_inline<kAppendInlineInts>(dtype, a, meta, n_meta, blocks, s);
+    else if (dtype == PA_KV_FP16) hipLaunchKernelGGL(append_batch_kernel<2>, dim3(blocks), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL(append_batch_kernel<1>, dim3(blocks), dim3(256), 0, s, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_stage_copy(const int32_t* host, int32_t* dev, size_t n, hipStream_t s) {
+    const int vecs = static_cast<int>((n + 3) / 4);
+    if (vecs == 0) return hipSuccess;
+    hipLaunchKernelGGL(stage_copy_kernel, dim3((vecs + 255) / 256), dim3(256), 0, s,
+                       reinterpret_cast<const u32x4*>(host), reinterpret_cast<u32x4*>(dev), vecs);
     return hipGetLastError();
 }
 

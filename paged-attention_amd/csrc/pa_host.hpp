@@ -30,6 +30,7 @@ struct pa_plan {
 // last stream operation that reads them.
 struct pa_stage {
     int32_t*   host = nullptr;
+    int32_t*   host_dev = nullptr;   // host, as kernels address it
     int32_t*   dev  = nullptr;
     size_t     cap  = 0;   // int32 elements
     hipEvent_t done = nullptr;
@@ -78,6 +79,12 @@ struct pa_pool {
     std::vector<char>                 occupied;
 };
 
+// The last append queued on a stream.
+struct pa_stream_mark {
+    hipStream_t stream = nullptr;
+    hipEvent_t  done   = nullptr;
+};
+
 struct pa_cache {
     pa_cache_config cfg{};
     pa_pool         pool;
@@ -89,7 +96,8 @@ struct pa_cache {
     pa_device_plan  dplan;                    // its extra ints are the plan's slot ids
     int             plan_batch = 0;
     int             plan_hq    = 0;
-    pa_stage_pool   append_staging;           // the batched append's metadata
+    pa_stage_pool   append_staging;           // appends' metadata past the kernel arguments' size
+    std::vector<pa_stream_mark> append_marks; // appends whose metadata went in the arguments
 };
 
 namespace pa::host {

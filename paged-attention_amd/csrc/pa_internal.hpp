@@ -88,7 +88,15 @@ struct AppendBatch {
     int             hkv, page_size;
     float           inv_k, inv_v;
 };
-hipError_t launch_append_batch(int dtype, const AppendBatch& a, hipStream_t s);
+// `meta` (host, n_meta ints) goes over inside the kernel's arguments when it
+// fits (append_meta_inline); else it is null and a.meta is on the device.
+hipError_t launch_append_batch(int dtype, const AppendBatch& a, const int32_t* meta, size_t n_meta, hipStream_t s);
+// Whether an append's meta of n ints fits the kernel arguments (4 KiB in all).
+constexpr size_t kAppendInlineInts = 896;
+constexpr bool   append_meta_inline(size_t n) { return n <= kAppendInlineInts; }
+// Copies n ints (rounded up to whole 16 bytes) from pinned host memory to the
+// device with a kernel. Both ends are 16-byte aligned and have that room.
+hipError_t launch_stage_copy(const int32_t* host, int32_t* dev, size_t n, hipStream_t s);
 hipError_t launch_gather(int dtype, const void* cache, const int32_t* bt_row, int hkv,
                          int page_size, int kv_head, int len, void* out, hipStream_t s);
 hipError_t launch_fill_bytes(void* buf, size_t bytes, int value, hipStream_t s);

@@ -36,6 +36,107 @@ void cache_params(const pa_cache& c, pa_decode_params& p) {
     p.v_scale            = fp8 ? c.cfg.v_scale : 1.0f;
 }
 
+// Records that an append was queued on s: one event per stream, moved on by
+// each further append there. Past kMaxMarks streams the oldest mark's stream is
+// waited for and its event taken over.
+void mark_append(pa_cache& c, hipStream_t s) {
+    constexpr size_t kMaxMarks = 8;
+    size_t i = 0;
+    while (i < c.append_marks.size() && c.append_marks[i].stream != s) ++i;
+    if (i == c.append_marks.size()) {
+        if (i < kMaxMarks) {
+            hipEvent_t ev = nullptr;
+            pa::hip_check(hipEventCreateWithFlags(&ev, hipEventDisableTiming), "hipEventCreate");
+            c.append_marks.push_back({s, ev});
+        } else {
+            std::rotate(c.append_marks.begin(), c.append_marks.begin() + 1, c.append_marks.end());
+            i = kMaxMarks - 1;
+            pa::hip_check(hipEventSynchronize(c.append_marks[i].done), "hipEventSynchronize append");
+            c.append_marks[i].stream = s;
+        }
+    }
+    pa::hip_check(hipEventRecord(c.append_marks[i].done, s), "hipEventRecord append");
+}
+
+// Queues one kernel that writes the tokens of reserved entries, the table
+// entries they added and the new lengths. Its meta (layout of
+// pa::AppendBatch::meta: per entry its first token, old length and page-list
+// start; the page lists; the new table entries; one (slot, length) per distinct
+// slot) goes over in the kernel's arguments when it fits, else through a staging
+// buffer and a copy kernel.
+void queue_append(pa_cache& c, const int32_t* slots, const int32_t* counts, int n,
+                  const std::vector<reserve_entry>& entries, long n_tok, const uint16_t* d_k, const uint16_t* d_v,
+                  hipStream_t s) {
+    const int P = c.cfg.page_size;
+    long n_tab = 0, n_pl = 0;
+    for (int i = 0; i < n; ++i) {
+        const reserve_entry& e = entries[static_cast<size_t>(i)];
+        n_tab += e.num_new;
+        if (counts[i] > 0) n_pl += (e.old_len + counts[i] - 1) / P - e.old_len / P + 1;
+    }
+    std::vector<char> seen(static_cast<size_t>(c.cfg.max_slots), 0);
+    long n_len = 0;
+    for (int i = 0; i < n; ++i)
+        if (!seen[static_cast<size_t>(slots[i])]) seen[static_cast<size_t>(slots[i])] = 1, ++n_len;
+    const size_t need = 3 * static_cast<size_t>(n) + static_cast<size_t>(n_pl) + 2 * static_cast<size_t>(n_tab + n_len);
+    const bool in_args = pa::append_meta_inline(need);
+    int32_t  args[pa::kAppendInlineInts];
+    pa_stage* st = in_args ? nullptr : &take_stage(c.append_staging, need, true);
+    int32_t* tok_begin = in_args ? args : st->host;
+    int32_t* const meta = tok_begin;
+    int32_t* old_len   = tok_begin + n;
+    int32_t* pl_begin  = old_len + n;
+    int32_t* pages     = pl_begin + n;
+    int32_t* tab       = pages + n_pl;
+    int32_t* lens      = tab + 2 * n_tab;
+    int32_t  tok = 0, pl = 0;
+    for (int i = 0; i < n; ++i) {
+        const auto& table = c.pool.tables[static_cast<size_t>(slots[i])];
+        const reserve_entry& e = entries[static_cast<size_t>(i)];
+        tok_begin[i] = tok;
+        old_len[i]   = e.old_len;
+        pl_begin[i]  = pl;
+        tok += counts[i];
+        if (counts[i] > 0)
+            for (int k = e.old_len / P; k <= (e.old_len + counts[i] - 1) / P; ++k) pages[pl++] = table[static_cast<size_t>(k)];
+        for (int k = e.first_new; k < e.first_new + e.num_new; ++k) {
+            *tab++ = slots[i] * c.cfg.max_pages_per_slot + k;
+            *tab++ = table[static_cast<size_t>(k)];
+        }
+    }
+    for (int i = 0; i < n; ++i) {
+        const size_t sl = static_cast<size_t>(slots[i]);
+        if (seen[sl] != 1) continue;
+        seen[sl] = 2;
+        *lens++ = slots[i];
+        *lens++ = c.pool.seq_lens[sl];
+    }
+    const bool fp8 = c.cfg.dtype == PA_KV_FP8_E4M3;
+    pa::AppendBatch a{};
+    a.k = d_k;
+    a.v = d_v;
+    a.k_cache = c.d_k;
+    a.v_cache = c.d_v;
+    a.meta = in_args ? nullptr : st->dev;
+    a.table = c.d_table;
+    a.seq_lens = c.d_seq_lens;
+    a.n_ent = n;
+    a.n_pl = static_cast<int>(n_pl);
+    a.n_tab = static_cast<int>(n_tab);
+    a.n_len = static_cast<int>(n_len);
+    a.n_tok = static_cast<int>(n_tok);
+    a.hkv = c.cfg.num_kv_heads;
+    a.page_size = P;
+    a.inv_k = fp8 ? 1.0f / c.cfg.k_scale : 1.0f;
+    a.inv_v = fp8 ? 1.0f / c.cfg.v_scale : 1.0f;
+    if (!in_args) pa::hip_check(pa::launch_stage_copy(st->host_dev, st->dev, need, s), "append staging kernel launch");
+    pa::hip_check(pa::launch_append_batch(c.cfg.dtype, a, in_args ? meta : nullptr, need, s), "append kernel launch");
+    // Tells a later use of the buffer, and release, when this append is done
+    // (release works on the null stream, which orders itself after its own work).
+    if (!in_args) release_stage(*st, s);
+    else if (s) mark_append(c, s);
+}
+
 void cache_plan(pa_cache& c, const int32_t* slots, int n, int hq, int num_ctas, hipStream_t s) {
     if (n < 0 || (n > 0 && !slots)) throw std::invalid_argument("plan: bad slot list");
     std::vector<int32_t> lens(static_cast<size_t>(n));
@@ -116,6 +217,7 @@ void pa_cache_destroy(pa_cache* c) {
     (void)hipFree(c->d_table);
     (void)hipFree(c->d_seq_lens);
     free_stages(c->append_staging);
+    for (pa_stream_mark& m : c->append_marks) (void)hipEventDestroy(m.done);
     device_plan_free(c->dplan);
     delete c;
 }
@@ -136,22 +238,8 @@ pa_status pa_cache_append(pa_cache* c, int slot, const uint16_t* d_k, const uint
         if (appended) *appended = 1;
         if (n <= 0) return;
         const hipStream_t s = as_stream(stream);
-        int32_t* row = c->d_table + static_cast<size_t>(slot) * c->cfg.max_pages_per_slot;
-        const auto& table = c->pool.tables[static_cast<size_t>(slot)];
-        if (num_new > 0)
-            pa::hip_check(hipMemcpyAsync(row + first_new, table.data() + first_new, sizeof(int32_t) * num_new,
-                                         hipMemcpyHostToDevice, s),
-                          "hipMemcpyAsync block table");
-        pa::hip_check(hipMemcpyAsync(c->d_seq_lens + slot, &c->pool.seq_lens[static_cast<size_t>(slot)],
-                                     sizeof(int32_t), hipMemcpyHostToDevice, s),
-                      "hipMemcpyAsync seq_len");
-        const bool fp8 = c->cfg.dtype == PA_KV_FP8_E4M3;
-        const float inv_k = fp8 ? 1.0f / c->cfg.k_scale : 1.0f;
-        const float inv_v = fp8 ? 1.0f / c->cfg.v_scale : 1.0f;
-        pa::hip_check(pa::launch_append(c->cfg.dtype, d_k, d_v, c->d_k, c->d_v, row, old_len, n, c->cfg.num_kv_heads,
-                                        c->cfg.page_size, inv_k, inv_v, s),
-                      "append kernel launch");
-        // The copies above read host memory the next call may change.
+        const std::vector<reserve_entry> entry{{old_len, first_new, num_new}};
+        queue_append(*c, &slot, &n, 1, entry, n, d_k, d_v, s);
         pa::hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
     });
 }
@@ -171,74 +259,7 @@ pa_status pa_cache_append_batch(pa_cache* c, const int32_t* slots, const int32_t
         if (appended) *appended = 1;
         if (n_tok == 0) return;
 
-        // Staging (layout of pa::AppendBatch::meta): per entry its first
-        // token, old length and page-list start; the page lists; the new table
-        // entries; one (slot, length) per distinct slot.
-        const int P = c->cfg.page_size;
-        long n_tab = 0, n_pl = 0;
-        for (int i = 0; i < n; ++i) {
-            const reserve_entry& e = entries[static_cast<size_t>(i)];
-            n_tab += e.num_new;
-            if (counts[i] > 0) n_pl += (e.old_len + counts[i] - 1) / P - e.old_len / P + 1;
-        }
-        std::vector<char> seen(static_cast<size_t>(c->cfg.max_slots), 0);
-        long n_len = 0;
-        for (int i = 0; i < n; ++i)
-            if (!seen[static_cast<size_t>(slots[i])]) seen[static_cast<size_t>(slots[i])] = 1, ++n_len;
-        const size_t need = 3 * static_cast<size_t>(n) + static_cast<size_t>(n_pl) + 2 * static_cast<size_t>(n_tab + n_len);
-        pa_stage& st = take_stage(c->append_staging, need, true);
-        int32_t* tok_begin = st.host;
-        int32_t* old_len   = tok_begin + n;
-        int32_t* pl_begin  = old_len + n;
-        int32_t* pages     = pl_begin + n;
-        int32_t* tab       = pages + n_pl;
-        int32_t* lens      = tab + 2 * n_tab;
-        int32_t  tok = 0, pl = 0;
-        for (int i = 0; i < n; ++i) {
-            const auto& table = c->pool.tables[static_cast<size_t>(slots[i])];
-            const reserve_entry& e = entries[static_cast<size_t>(i)];
-            tok_begin[i] = tok;
-            old_len[i]   = e.old_len;
-            pl_begin[i]  = pl;
-            tok += counts[i];
-            if (counts[i] > 0)
-                for (int k = e.old_len / P; k <= (e.old_len + counts[i] - 1) / P; ++k) pages[pl++] = table[static_cast<size_t>(k)];
-            for (int k = e.first_new; k < e.first_new + e.num_new; ++k) {
-                *tab++ = slots[i] * c->cfg.max_pages_per_slot + k;
-                *tab++ = table[static_cast<size_t>(k)];
-            }
-        }
-        for (int i = 0; i < n; ++i) {
-            const size_t sl = static_cast<size_t>(slots[i]);
-            if (seen[sl] != 1) continue;
-            seen[sl] = 2;
-            *lens++ = slots[i];
-            *lens++ = c->pool.seq_lens[sl];
-        }
-
-        const hipStream_t s = as_stream(stream);
-        pa::hip_check(hipMemcpyAsync(st.dev, st.host, need * sizeof(int32_t), hipMemcpyHostToDevice, s),
-                      "hipMemcpyAsync append staging");
-        const bool fp8 = c->cfg.dtype == PA_KV_FP8_E4M3;
-        pa::AppendBatch a{};
-        a.k = d_k;
-        a.v = d_v;
-        a.k_cache = c->d_k;
-        a.v_cache = c->d_v;
-        a.meta = st.dev;
-        a.table = c->d_table;
-        a.seq_lens = c->d_seq_lens;
-        a.n_ent = n;
-        a.n_pl = static_cast<int>(n_pl);
-        a.n_tab = static_cast<int>(n_tab);
-        a.n_len = static_cast<int>(n_len);
-        a.n_tok = static_cast<int>(n_tok);
-        a.hkv = hkv;
-        a.page_size = P;
-        a.inv_k = fp8 ? 1.0f / c->cfg.k_scale : 1.0f;
-        a.inv_v = fp8 ? 1.0f / c->cfg.v_scale : 1.0f;
-        pa::hip_check(pa::launch_append_batch(c->cfg.dtype, a, s), "append_batch kernel launch");
-        release_stage(st, s);
+        queue_append(*c, slots, counts, n, entries, n_tok, d_k, d_v, as_stream(stream));
     });
 }
 
@@ -249,6 +270,8 @@ pa_status pa_cache_release(pa_cache* c, int slot) {
         // A batched append still in flight may write this slot's length.
         for (pa_stage& st : c->append_staging.bufs)
             if (st.done) pa::hip_check(hipEventSynchronize(st.done), "hipEventSynchronize staging");
+        for (pa_stream_mark& m : c->append_marks)
+            pa::hip_check(hipEventSynchronize(m.done), "hipEventSynchronize append");
         pa::hip_check(hipMemset(c->d_seq_lens + slot, 0, sizeof(int32_t)), "hipMemset seq_len");
     });
 }

@@ -196,14 +196,16 @@ pa_stage& take_stage(pa_stage_pool& sp, size_t need, bool with_device) {
     sp.next = (pick + 1) % sp.bufs.size();
     pa_stage& st = sp.bufs[pick];
     if (st.cap < need || (with_device && !st.dev)) {
-        const size_t cap = std::max<size_t>(need + need / 2, 4096);
+        const size_t cap = (std::max<size_t>(need + need / 2, 4096) + 3) & ~size_t{3};   // whole 16 bytes
         (void)hipHostFree(st.host);
         (void)hipFree(st.dev);
         st.host = nullptr;
         st.dev  = nullptr;
         st.cap  = 0;
-        pa::hip_check(hipHostMalloc(reinterpret_cast<void**>(&st.host), cap * sizeof(int32_t), hipHostMallocDefault),
+        pa::hip_check(hipHostMalloc(reinterpret_cast<void**>(&st.host), cap * sizeof(int32_t), hipHostMallocMapped),
                       "hipHostMalloc staging");
+        pa::hip_check(hipHostGetDevicePointer(reinterpret_cast<void**>(&st.host_dev), st.host, 0),
+                      "hipHostGetDevicePointer staging");
         if (with_device)
             pa::hip_check(hipMalloc(reinterpret_cast<void**>(&st.dev), cap * sizeof(int32_t)), "hipMalloc staging");
         st.cap = cap;
@@ -270,8 +272,7 @@ void device_plan_upload(pa_device_plan& dp, const pa_plan& plan, int group, int 
     if (n_extra) std::copy(extra, extra + n_extra, st.host + o_extra);
     std::fill(st.host + o_ctr, st.host + o_unit, 0);
     if (blocks) std::copy(item_unit.begin(), item_unit.end(), st.host + o_unit);
-    pa::hip_check(hipMemcpyAsync(dp.ints, st.host, total * sizeof(int32_t), hipMemcpyHostToDevice, s),
-                  "hipMemcpyAsync plan");
+    pa::hip_check(pa::launch_stage_copy(st.host_dev, dp.ints, total, s), "plan upload kernel launch");
     release_stage(st, s);
     dp.segments       = dp.ints;
     dp.cta_seg_begin  = dp.ints + o_cta;
