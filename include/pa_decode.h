@@ -332,6 +332,10 @@ pa_status pa_cache_append(pa_cache* cache, int slot, const uint16_t* d_k, const 
  * still in flight. */
 pa_status pa_cache_append_batch(pa_cache* cache, const int32_t* slots, const int32_t* counts, int n,
                                 const uint16_t* d_k, const uint16_t* d_v, void* stream, int* appended);
+/* paged_kv_cache.cu:138-146 release. The slot's length on the device becomes
+ * zero in order with the cache's other work: queued on the null stream where
+ * every call so far was given that (the call does not wait), else before the
+ * call returns. */
 pa_status pa_cache_release(pa_cache* cache, int slot);
 void      pa_cache_shuffle_free_pages(pa_cache* cache, unsigned seed);
 /* paged_kv_cache.cu:157-171 params(): cache-side fields of DecodeParams. */

@@ -272,15 +272,25 @@ __global__ __launch_bounds__(256) void append_inline_kernel(const AppendInline<N
     append_batch_body<EB>(x.a, reinterpret_cast<const int32_t*>(args + offsetof(AppendInline<N>, meta)));
 }
 
+__global__ void zero_int_kernel(int32_t* p) { *p = 0; }
+
 // Pinned host memory to the device, 16 bytes per thread. Bound by the bus and
 // its latency (56 KB of a 2048-unit plan: 4.0 us). The runtime's copy took 6.3
 // us on a DMA engine plus the decode's wait for another queue, and a new
 // request's host step more than a launch: with this and the arguments' meta
 // above, a step of 30 resident and 2 joining sequences 94.6 -> 85.0 us, of 16
 // and 1 (one-sequence append) 71.9 -> 60.4.
-__global__ __launch_bounds__(256) void stage_copy_kernel(const u32x4* __restrict__ host, u32x4* __restrict__ dev, int n) {
+__global__ __launch_bounds__(256) void stage_copy_kernel(const u32x4* __restrict__ host, u32x4* __restrict__ dev, int n,
+                                                         int32_t* marks, int32_t mark) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) dev[i] = host[i];
+    if (marks) {
+        // Every thread's load has returned before the block's mark goes out.
+        __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
+        __syncthreads();
+        if (threadIdx.x == 0)
+            __hip_atomic_store(marks + blockIdx.x, mark, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
 }
 
 // One thread per (token, 8-dim chunk) of one kv head: raw cache bytes out,
@@ -414,11 +424,16 @@ hipError_t launch_append_batch(int dtype, const AppendBatch& a, const int32_t* m
     return hipGetLastError();
 }
 
-hipError_t launch_stage_copy(const int32_t* host, int32_t* dev, size_t n, hipStream_t s) {
+hipError_t launch_zero_int(int32_t* p, hipStream_t s) {
+    hipLaunchKernelGGL(zero_int_kernel, dim3(1), dim3(1), 0, s, p);
+    return hipGetLastError();
+}
+
+hipError_t launch_stage_copy(const int32_t* host, int32_t* dev, size_t n, int32_t* marks, int32_t mark, hipStream_t s) {
     const int vecs = static_cast<int>((n + 3) / 4);
     if (vecs == 0) return hipSuccess;
-    hipLaunchKernelGGL(stage_copy_kernel, dim3((vecs + 255) / 256), dim3(256), 0, s,
-                       reinterpret_cast<const u32x4*>(host), reinterpret_cast<u32x4*>(dev), vecs);
+    hipLaunchKernelGGL(stage_copy_kernel, dim3(static_cast<unsigned>(stage_copy_blocks(n))), dim3(256), 0, s,
+                       reinterpret_cast<const u32x4*>(host), reinterpret_cast<u32x4*>(dev), vecs, marks, mark);
     return hipGetLastError();
 }
 

@@ -15,6 +15,17 @@
 #include <string>
 #include <vector>
 
+// How a plan's split items lie in units and blocks.
+struct pa_split_shape {
+    bool split        = false;   // some item has several segments
+    bool slots        = true;    // every split segment is its unit's first or last
+    bool in_block     = true;    // no item spans blocks
+    bool consecutive  = true;    // an item's k-th segment runs in unit u0 + k
+    int  max_blocks   = 0;       // most blocks of one split item
+    int  max_segments = 0;       // most segments of one item
+    std::vector<int32_t> item_unit;   // [items] unit of each item's first segment
+};
+
 // Host copy of a schedule (decode.hpp:21-27 DecodePlan).
 struct pa_plan {
     int num_ctas = 0;
@@ -23,16 +34,21 @@ struct pa_plan {
     std::vector<int32_t> segments;        // [n][4] = (row, kv head, tok_begin, tok_end)
     std::vector<int32_t> cta_seg_begin;   // [num_ctas + 1]
     std::vector<int32_t> item_seg_begin;  // [items + 1]
+    pa_split_shape       shape;
 };
 
 // One pinned host staging buffer for host-to-device copies on a stream: pinned
-// host ints, optionally their own device copy, and an event recorded after the
-// last stream operation that reads them.
+// host ints, optionally their own device copy, and what tells when the last
+// stream operation that reads them is done: marks that the copy kernel leaves
+// behind the ints, or an event.
 struct pa_stage {
     int32_t*   host = nullptr;
     int32_t*   host_dev = nullptr;   // host, as kernels address it
     int32_t*   dev  = nullptr;
-    size_t     cap  = 0;   // int32 elements
+    size_t     cap  = 0;   // int32 elements, marks not counted
+    size_t     marks = 0;  // marks of the last copy (at host + cap), one per block
+    int32_t    mark  = 0;  // their value once it has read the buffer
+    bool       captured = false;   // a graph's copy kernel reads it: kept as it is until the pool goes
     hipEvent_t done = nullptr;
 };
 
@@ -98,6 +114,8 @@ struct pa_cache {
     int             plan_hq    = 0;
     pa_stage_pool   append_staging;           // appends' metadata past the kernel arguments' size
     std::vector<pa_stream_mark> append_marks; // appends whose metadata went in the arguments
+    bool            null_stream_only = true;  // no call was given another stream yet
+    bool            zero_queued = false;      // a release's zero length may still be queued on the null stream
 };
 
 namespace pa::host {
@@ -140,6 +158,10 @@ inline hipStream_t as_stream(void* s) { return static_cast<hipStream_t>(s); }
 pa_stage& take_stage(pa_stage_pool& sp, size_t need, bool with_device);
 // Records the buffer's event on s: call after queuing the work that reads it.
 void release_stage(pa_stage& st, hipStream_t s);
+// Queues the copy kernel of the buffer's first n ints to dev, which marks the
+// buffer as read: no event. (An event between two kernels of a stream costs 4 us
+// of the stream's time.)
+void copy_stage(pa_stage& st, int32_t* dev, size_t n, hipStream_t s);
 // Waits for every queued use of the pool and frees its buffers and events.
 void free_stages(pa_stage_pool& sp);
 

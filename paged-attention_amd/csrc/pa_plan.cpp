@@ -9,6 +9,7 @@
 #include <algorithm>
 #include <climits>
 #include <string>
+#include <thread>
 #include <vector>
 
 namespace {
@@ -40,6 +41,10 @@ int wave_ctas_impl(int dtype, int head_dim, int group) {
     return device_cus() * pa::kernel_units_per_cu(dtype, group);
 }
 
+// Segments of one item whose partial rows the kernels address with 32-bit
+// offsets (8 heads x 128 floats each).
+constexpr int kMaxItemSegments = 1 << 19;
+
 // The persistent cut (decode.cu:65-108): all (row, kv head) items are laid out
 // in order as runs of `tile`-token tiles; the total is split into equal
 // contiguous ranges of `per` tiles, one per work unit, and every maximal run of
@@ -49,50 +54,77 @@ void cut(pa_plan& plan, int tile, const int32_t* lens, int batch, int hkv, int r
     if (batch < 0 || hkv <= 0) throw std::invalid_argument("make_plan: bad batch or kv head count");
     if (batch > 0 && !lens) throw std::invalid_argument("make_plan: seq_lens is null");
     if (requested <= 0) throw std::invalid_argument("make_plan: num_ctas must be positive");
-    plan = pa_plan{};
-    plan.tile  = tile;
-    plan.items = batch * hkv;
+    // Emptied (its arrays' memory stays for the next cut), also when a length
+    // is refused.
+    plan.segments.clear();
+    plan.cta_seg_begin.clear();
+    plan.item_seg_begin.clear();
+    plan.shape    = {};
+    plan.num_ctas = 0;
+    plan.tile     = tile;
+    plan.items    = batch * hkv;
 
-    std::vector<long> tiles_of(static_cast<size_t>(batch));
     long total = 0;
     for (int b = 0; b < batch; ++b) {
         if (lens[b] <= 0) throw std::invalid_argument("make_plan: every sequence needs at least one token");
-        tiles_of[b] = (static_cast<long>(lens[b]) + tile - 1) / tile;
-        total += tiles_of[b] * hkv;
+        total += (static_cast<long>(lens[b]) + tile - 1) / tile * hkv;
     }
     plan.item_seg_begin.assign(static_cast<size_t>(plan.items) + 1, 0);
-    if (total == 0) {
-        plan.cta_seg_begin.push_back(0);
-        return;
-    }
+    plan.cta_seg_begin.assign(1, 0);
+    if (total == 0) return;
     const long per = (total + requested - 1) / requested;
     plan.num_ctas = static_cast<int>((total + per - 1) / per);
-    plan.cta_seg_begin.reserve(static_cast<size_t>(plan.num_ctas) + 1);
+    plan.cta_seg_begin.resize(static_cast<size_t>(plan.num_ctas) + 1);
+    // Every unit boundary adds at most one segment to the items' own.
+    plan.segments.resize(4 * (static_cast<size_t>(plan.num_ctas) + static_cast<size_t>(plan.items)));
+    pa_split_shape& sh = plan.shape;
+    sh.item_unit.resize(static_cast<size_t>(plan.items));
 
-    int  item = 0;
-    long done = 0;   // tiles of `item` already assigned
-    for (int u = 0; u < plan.num_ctas; ++u) {
-        plan.cta_seg_begin.push_back(static_cast<int32_t>(plan.segments.size() / 4));
-        long budget = per;
-        while (budget > 0 && item < plan.items) {
-            const int  b     = item / hkv;
-            const long avail = tiles_of[b] - done;
-            const long take  = std::min(budget, avail);
-            const long t0    = done * tile;
-            const long t1    = std::min((done + take) * tile, static_cast<long>(lens[b]));
-            plan.segments.insert(plan.segments.end(),
-                                 {b, item % hkv, static_cast<int32_t>(t0), static_cast<int32_t>(t1)});
-            plan.item_seg_begin[static_cast<size_t>(item) + 1] += 1;
-            done += take;
-            budget -= take;
-            if (done == tiles_of[b]) {
-                ++item;
-                done = 0;
+    int32_t* seg  = plan.segments.data();
+    int32_t  nseg = 0;
+    int      item = 0, u = 0;   // u: the current unit
+    long     left = per;        // tiles the current unit still takes
+    for (int b = 0; b < batch; ++b) {
+        const long tiles = (static_cast<long>(lens[b]) + tile - 1) / tile;
+        for (int h = 0; h < hkv; ++h, ++item) {
+            const int32_t first = nseg;
+            plan.item_seg_begin[static_cast<size_t>(item)] = first;
+            if (left == 0) {
+                plan.cta_seg_begin[static_cast<size_t>(++u)] = nseg;
+                left = per;
+            }
+            sh.item_unit[static_cast<size_t>(item)] = u;
+            for (long done = 0; done < tiles;) {
+                if (left == 0) {
+                    plan.cta_seg_begin[static_cast<size_t>(++u)] = nseg;
+                    left = per;
+                }
+                const long take = std::min(left, tiles - done);
+                seg[0] = b;
+                seg[1] = h;
+                seg[2] = static_cast<int32_t>(done * tile);
+                seg[3] = static_cast<int32_t>(std::min((done + take) * tile, static_cast<long>(lens[b])));
+                seg += 4;
+                ++nseg;
+                done += take;
+                left -= take;
+            }
+            // What split_shape would find: a unit takes one run of an item, and
+            // an item's runs lie in consecutive units.
+            const int n = nseg - first;
+            sh.max_segments = std::max(sh.max_segments, n);
+            if (n > 1) {
+                const int nb = u / pa::kBlockUnits - sh.item_unit[static_cast<size_t>(item)] / pa::kBlockUnits + 1;
+                sh.split      = true;
+                sh.max_blocks = std::max(sh.max_blocks, nb);
+                if (nb > 1) sh.in_block = false;
+                if (n >= kMaxItemSegments) sh.consecutive = false;
             }
         }
     }
-    plan.cta_seg_begin.push_back(static_cast<int32_t>(plan.segments.size() / 4));
-    for (int i = 0; i < plan.items; ++i) plan.item_seg_begin[i + 1] += plan.item_seg_begin[i];
+    plan.item_seg_begin[static_cast<size_t>(plan.items)] = nseg;
+    plan.cta_seg_begin[static_cast<size_t>(plan.num_ctas)] = nseg;
+    plan.segments.resize(4 * static_cast<size_t>(nseg));
 }
 
 }  // namespace
@@ -105,33 +137,26 @@ void check_dtype(int dtype) {
     if (dtype != PA_KV_FP16 && dtype != PA_KV_FP8_E4M3)
         throw std::invalid_argument("unknown kv dtype " + std::to_string(dtype));
 }
-// How a plan's split items lie in units and blocks.
-struct SplitShape {
-    bool split       = false;   // some item has several segments
-    bool slots       = true;    // every split segment is its unit's first or last
-    bool in_block    = true;    // no item spans blocks
-    bool consecutive = true;    // an item's k-th segment runs in unit u0 + k
-    int  max_blocks  = 0;       // most blocks of one split item
-};
-SplitShape split_shape(const pa_plan& plan, std::vector<int32_t>* item_unit) {
-    SplitShape sh;
+// The shape of any plan, from its arrays (make_plan's cut fills its own).
+pa_split_shape split_shape(const pa_plan& plan) {
+    pa_split_shape sh;
     const size_t nseg = plan.segments.size() / 4;
     sh.split = nseg > static_cast<size_t>(plan.items);
-    if (!sh.split) return sh;
     std::vector<int32_t> unit_of(nseg, 0);
     for (int u = 0; u < plan.num_ctas; ++u)
         for (int sg = plan.cta_seg_begin[u]; sg < plan.cta_seg_begin[u + 1]; ++sg)
             unit_of[static_cast<size_t>(sg)] = u;
-    if (item_unit) item_unit->resize(static_cast<size_t>(plan.items));
+    sh.item_unit.resize(static_cast<size_t>(plan.items));
     for (int i = 0; i < plan.items; ++i) {
         const int a = plan.item_seg_begin[i], z = plan.item_seg_begin[i + 1];
         const int u0 = unit_of[static_cast<size_t>(a)];
-        if (item_unit) (*item_unit)[static_cast<size_t>(i)] = u0;
+        sh.item_unit[static_cast<size_t>(i)] = u0;
+        sh.max_segments = std::max(sh.max_segments, z - a);
         if (z - a <= 1) continue;
         const int nb = unit_of[static_cast<size_t>(z - 1)] / pa::kBlockUnits - u0 / pa::kBlockUnits + 1;
         sh.max_blocks = std::max(sh.max_blocks, nb);
         if (nb > 1) sh.in_block = false;
-        if (z - a >= (1 << 19)) sh.consecutive = false;   // 32-bit offsets of 8 heads x 128 floats
+        if (z - a >= kMaxItemSegments) sh.consecutive = false;
         for (int sg = a; sg < z; ++sg) {
             const int u = unit_of[static_cast<size_t>(sg)];
             if (sg != plan.cta_seg_begin[u] && sg != plan.cta_seg_begin[u + 1] - 1) sh.slots = false;
@@ -153,7 +178,7 @@ constexpr int kChainMaxBlocks = 8;
 // with; 1 x 16384 fp16 14.7 / 15.1; 2 x 16384 FP8 level) until an item has
 // hundreds of segments (one kv head, 1 x 131072 fp16, 256 blocks: 18.2 / 15.6).
 constexpr int kOneHeadMinBlocks = 64;
-int merge_mode_of(const SplitShape& sh, int max_blocks) {
+int merge_mode_of(const pa_split_shape& sh, int max_blocks) {
     // The split kernel keeps a unit's split segments in two LDS slots: they
     // must be the unit's first and last segments (true of every make_plan cut).
     if (!sh.split || !sh.slots) return 0;
@@ -166,7 +191,7 @@ int merge_mode_of(const SplitShape& sh, int max_blocks) {
 #endif
     return 0;
 }
-int plan_merge_mode(const pa_plan& plan) { return merge_mode_of(split_shape(plan, nullptr), kChainMaxBlocks); }
+int plan_merge_mode(const pa_plan& plan) { return merge_mode_of(plan.shape, kChainMaxBlocks); }
 void make_plan_impl(pa_plan& plan, int dtype, const int32_t* lens, int batch, int hq, int hkv, int hd,
                     int num_ctas) {
     const int group = group_of(hq, hkv);
@@ -175,46 +200,86 @@ void make_plan_impl(pa_plan& plan, int dtype, const int32_t* lens, int batch, in
     if (num_ctas <= 0) num_ctas = wave_ctas_impl(dtype, hd, group);
     cut(plan, tile, lens, batch, hkv, num_ctas);
 }
+namespace {
+// Whether the copy kernel of the buffer's last use has read it.
+bool stage_read(const pa_stage& st) {
+    for (size_t i = 0; i < st.marks; ++i)
+        if (__atomic_load_n(st.host + st.cap + i, __ATOMIC_ACQUIRE) != st.mark) return false;
+    return true;
+}
+bool stage_idle(const pa_stage& st) {
+    if (!stage_read(st)) return false;
+    if (!st.done) return true;
+    const hipError_t q = hipEventQuery(st.done);
+    if (q != hipErrorNotReady) pa::hip_check(q, "hipEventQuery staging");
+    return q == hipSuccess;
+}
+}  // namespace
 pa_stage& take_stage(pa_stage_pool& sp, size_t need, bool with_device) {
     const size_t n = sp.bufs.size();
-    size_t pick = n;
+    size_t pick = n, used = 0, oldest = n;
     for (size_t k = 0; k < n && pick == n; ++k) {
         const size_t i = (sp.next + k) % n;
-        const hipError_t q = hipEventQuery(sp.bufs[i].done);
-        if (q == hipSuccess) pick = i;
-        else if (q != hipErrorNotReady) pa::hip_check(q, "hipEventQuery staging");
+        if (sp.bufs[i].captured) continue;
+        ++used;
+        if (oldest == n) oldest = i;
+        if (stage_idle(sp.bufs[i])) pick = i;
     }
     if (pick == n) {
-        if (n < pa_stage_pool::kMaxStages) {
+        if (used < pa_stage_pool::kMaxStages) {
             sp.bufs.emplace_back();
-            pa::hip_check(hipEventCreateWithFlags(&sp.bufs.back().done, hipEventDisableTiming), "hipEventCreate");
         } else {
-            pick = sp.next % n;   // every buffer in flight: the oldest
-            pa::hip_check(hipEventSynchronize(sp.bufs[pick].done), "hipEventSynchronize staging");
+            pick = oldest;   // every buffer in flight
+            while (!stage_read(sp.bufs[pick])) std::this_thread::yield();
+            if (sp.bufs[pick].done)
+                pa::hip_check(hipEventSynchronize(sp.bufs[pick].done), "hipEventSynchronize staging");
         }
     }
     sp.next = (pick + 1) % sp.bufs.size();
     pa_stage& st = sp.bufs[pick];
     if (st.cap < need || (with_device && !st.dev)) {
         const size_t cap = (std::max<size_t>(need + need / 2, 4096) + 3) & ~size_t{3};   // whole 16 bytes
+        const size_t all = cap + pa::stage_copy_blocks(cap);
         (void)hipHostFree(st.host);
         (void)hipFree(st.dev);
-        st.host = nullptr;
-        st.dev  = nullptr;
-        st.cap  = 0;
-        pa::hip_check(hipHostMalloc(reinterpret_cast<void**>(&st.host), cap * sizeof(int32_t), hipHostMallocMapped),
+        st.host  = nullptr;
+        st.dev   = nullptr;
+        st.cap   = 0;
+        st.marks = 0;
+        pa::hip_check(hipHostMalloc(reinterpret_cast<void**>(&st.host), all * sizeof(int32_t),
+                                    hipHostMallocMapped | hipHostMallocCoherent),
                       "hipHostMalloc staging");
         pa::hip_check(hipHostGetDevicePointer(reinterpret_cast<void**>(&st.host_dev), st.host, 0),
                       "hipHostGetDevicePointer staging");
+        std::fill(st.host + cap, st.host + all, 0);
+        st.mark = 0;
         if (with_device)
             pa::hip_check(hipMalloc(reinterpret_cast<void**>(&st.dev), cap * sizeof(int32_t)), "hipMalloc staging");
         st.cap = cap;
     }
     return st;
 }
-void release_stage(pa_stage& st, hipStream_t s) { pa::hip_check(hipEventRecord(st.done, s), "hipEventRecord staging"); }
+void release_stage(pa_stage& st, hipStream_t s) {
+    if (!st.done) pa::hip_check(hipEventCreateWithFlags(&st.done, hipEventDisableTiming), "hipEventCreate");
+    pa::hip_check(hipEventRecord(st.done, s), "hipEventRecord staging");
+}
+void copy_stage(pa_stage& st, int32_t* dev, size_t n, hipStream_t s) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (s) pa::hip_check(hipStreamIsCapturing(s, &cs), "hipStreamIsCapturing");
+    if (cs != hipStreamCaptureStatusNone) {   // the graph's replays read it
+        pa::hip_check(pa::launch_stage_copy(st.host_dev, dev, n, nullptr, 0, s), "staging copy kernel launch");
+        st.captured = true;
+        return;
+    }
+    st.mark  = st.mark == INT32_MAX ? 1 : st.mark + 1;
+    st.marks = pa::stage_copy_blocks(n);
+    const hipError_t e = pa::launch_stage_copy(st.host_dev, dev, n, st.host_dev + st.cap, st.mark, s);
+    if (e != hipSuccess) st.marks = 0;   // nothing was queued
+    pa::hip_check(e, "staging copy kernel launch");
+}
 void free_stages(pa_stage_pool& sp) {
     for (pa_stage& st : sp.bufs) {
+        while (!stage_read(st)) std::this_thread::yield();
         if (st.done) (void)hipEventSynchronize(st.done);
         (void)hipHostFree(st.host);
         (void)hipFree(st.dev);
@@ -241,8 +306,7 @@ void device_plan_upload(pa_device_plan& dp, const pa_plan& plan, int group, int 
     const size_t o_item  = o_cta + round4(plan.cta_seg_begin.size());
     const size_t o_extra = o_item + round4(plan.item_seg_begin.size());
     const size_t o_ctr   = o_extra + round4(n_extra);   // per-item merge counters, uploaded as zeros
-    std::vector<int32_t> item_unit;
-    const SplitShape shape = split_shape(plan, &item_unit);
+    const pa_split_shape& shape = plan.shape;
     const int  in_kernel = merge_mode_of(shape, kChainMaxBlocks);
     // Past kChainMaxBlocks: block partials for the merge kernel (block_merge 3),
     // where the split kernel can find an item's part of a block. Same box, us per
@@ -252,7 +316,7 @@ void device_plan_upload(pa_device_plan& dp, const pa_plan& plan, int group, int 
     const bool blocks    = in_kernel == 0 && merge_mode_of(shape, INT_MAX) == 2 &&
                         (group > 1 || shape.max_blocks >= kOneHeadMinBlocks);
     const size_t o_unit  = o_ctr + pa::plan_item_units(plan.items);
-    const size_t total   = blocks ? o_unit + round4(item_unit.size()) : o_unit;
+    const size_t total   = blocks ? o_unit + round4(shape.item_unit.size()) : o_unit;
     if (total > dp.ints_cap) {
         // Growing frees the old block, which decodes queued before may still
         // read: wait for them first (growth only happens for a plan larger
@@ -271,9 +335,8 @@ void device_plan_upload(pa_device_plan& dp, const pa_plan& plan, int group, int 
     std::copy(plan.item_seg_begin.begin(), plan.item_seg_begin.end(), st.host + o_item);
     if (n_extra) std::copy(extra, extra + n_extra, st.host + o_extra);
     std::fill(st.host + o_ctr, st.host + o_unit, 0);
-    if (blocks) std::copy(item_unit.begin(), item_unit.end(), st.host + o_unit);
-    pa::hip_check(pa::launch_stage_copy(st.host_dev, dp.ints, total, s), "plan upload kernel launch");
-    release_stage(st, s);
+    if (blocks) std::copy(shape.item_unit.begin(), shape.item_unit.end(), st.host + o_unit);
+    copy_stage(st, dp.ints, total, s);
     dp.segments       = dp.ints;
     dp.cta_seg_begin  = dp.ints + o_cta;
     dp.item_seg_begin = dp.ints + o_item;
@@ -293,9 +356,7 @@ void device_plan_upload(pa_device_plan& dp, const pa_plan& plan, int group, int 
     dp.num_segments = static_cast<int>(nseg);
     dp.block_merge = blocks ? 3 : in_kernel;
     dp.needs_merge = blocks || (in_kernel == 0 && shape.split) ? 1 : 0;
-    dp.max_item_segments = 0;
-    for (int i = 0; i < plan.items; ++i)
-        dp.max_item_segments = std::max(dp.max_item_segments, plan.item_seg_begin[i + 1] - plan.item_seg_begin[i]);
+    dp.max_item_segments = shape.max_segments;
 }
 void device_plan_bind(const pa_device_plan& dp, pa_decode_params& p) {
     p.segments       = dp.segments;
@@ -425,6 +486,7 @@ pa_status pa_plan_create(int num_ctas, int tile, const int32_t* segments, int nu
         plan->segments.assign(segments, segments + 4 * static_cast<size_t>(num_segments));
         plan->cta_seg_begin.assign(cta_seg_begin, cta_seg_begin + num_ctas + 1);
         plan->item_seg_begin.assign(item_seg_begin, item_seg_begin + num_items + 1);
+        plan->shape    = split_shape(*plan);
         *out = plan;
     });
 }

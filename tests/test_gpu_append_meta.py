@@ -47,3 +47,77 @@ def test_appends_on_many_streams_then_release():
         t = cache.block_table(s)
         assert list(table[i, :len(t)]) == list(t)
     cache.close()
+
+
+def test_releases_on_the_null_stream_then_appends_on_another():
+    """Releases queued on the null stream (behind a long kernel there) and slots re-admitted at once, their
+    appends on a side stream: the new lengths stand, on the device too."""
+    import torch
+    P, hkv = 4, 2
+    cache = pa_amd.PagedKVCache(64, P, hkv, D, 3, 20)
+    x = torch.randn((50, hkv, D), dtype=torch.float16, device="cuda")
+    for i in range(3):
+        assert cache.append_batch([cache.admit()], [10 + i], x, x, 0)
+    big = torch.randn((4096, 4096), device="cuda")
+    torch.cuda.synchronize()
+    for _ in range(20):
+        big = big @ big
+        big = big / big.norm()
+    cache.release(0)
+    cache.release(2)
+    side = torch.cuda.Stream()
+    a, b = cache.admit(), cache.admit()
+    assert (a, b) == (0, 2)
+    assert cache.append_batch([a, b], [7, 9], x, x, side)
+    torch.cuda.synchronize()
+    assert list(d2h(cache.params().seq_lens, 12, np.int32)) == [7, 11, 9]
+    cache.release(1)   # now with another stream seen: zero when the call returns
+    assert list(d2h(cache.params().seq_lens, 12, np.int32)) == [7, 0, 9]
+    cache.close()
+
+
+def test_uploads_beyond_the_staging_buffers_and_in_a_graph():
+    """More plan uploads than staging buffers queued without a wait, each decode under its own plan; and an
+    upload captured into a graph with its decode, replayed between eager uploads of other plans."""
+    import torch
+    from helpers import paged_inputs
+    lens_of = [[64 * (i + 1), 5, 300 + i] for i in range(20)]
+    q, k, v, table, ks, vs = paged_inputs(3, [2000] * 3, 8, 2, 16, False, seed=3)
+    dplan = pa_amd.DevicePlan()
+
+    def decode(lens, out, stream=None, plan=None):
+        dplan.upload(plan or pa_amd.make_plan(pa_amd.FP16, lens, 8, 2, D), 4, D, stream)
+        p = pa_amd.DecodeParams()
+        p.q, p.k_cache, p.v_cache, p.block_table = q.data_ptr(), k.data_ptr(), v.data_ptr(), table.data_ptr()
+        p.out, p.block_table_stride = out.data_ptr(), table.size(1)
+        p.batch, p.num_q_heads, p.num_kv_heads, p.head_dim, p.page_size = 3, 8, 2, D, 16
+        p.sm_scale, p.k_scale, p.v_scale = pa_amd.sm_scale(D), ks, vs
+        dplan.bind(p)
+        pa_amd.paged_decode(pa_amd.FP16, p, stream)
+
+    largest = torch.empty_like(q)
+    decode([2000] * 3, largest)                      # sizes the plan's device arrays
+    plans = [pa_amd.make_plan(pa_amd.FP16, lens, 8, 2, D) for lens in lens_of]
+    alone = []
+    for lens in lens_of:
+        alone.append(torch.empty_like(q))
+        decode(lens, alone[-1])
+        torch.cuda.synchronize()
+    outs = [torch.empty_like(q) for _ in lens_of]
+    for lens, o, pl in zip(lens_of, outs, plans):
+        decode(lens, o, plan=pl)
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, o) for a, o in zip(alone, outs))
+    side, graph, out = torch.cuda.Stream(), torch.cuda.CUDAGraph(), torch.empty_like(q)
+    with torch.cuda.stream(side):
+        with torch.cuda.graph(graph, stream=side):
+            decode(lens_of[7], out, torch.cuda.current_stream(), plans[7])
+        for rep in range(3):
+            out.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, alone[7])
+            for i in range(12):
+                decode(lens_of[i], outs[i], side, plans[i])
+            torch.cuda.synchronize()
+            assert all(torch.equal(alone[i], outs[i]) for i in range(12))
