@@ -35,6 +35,7 @@ struct pa_plan {
     std::vector<int32_t> cta_seg_begin;   // [num_ctas + 1]
     std::vector<int32_t> item_seg_begin;  // [items + 1]
     pa_split_shape       shape;
+    int per = 0;   // tiles per unit if the plan is an equal cut as make_plan's, else 0
 };
 
 // One pinned host staging buffer for host-to-device copies on a stream: pinned
@@ -81,6 +82,7 @@ struct pa_device_plan {
     int      num_segments = 0;
     int      block_merge = 0;          // pa_decode_params.block_merge of the plan
     int32_t* merge_counters = nullptr;  // per-item counters in `ints`
+    pa_plan  blocks;                    // the plan cut again inside blocks, where that is what runs
     pa_stage_pool staging;
 };
 

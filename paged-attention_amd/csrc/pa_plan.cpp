@@ -63,6 +63,7 @@ void cut(pa_plan& plan, int tile, const int32_t* lens, int batch, int hkv, int r
     plan.num_ctas = 0;
     plan.tile     = tile;
     plan.items    = batch * hkv;
+    plan.per      = 0;
 
     long total = 0;
     for (int b = 0; b < batch; ++b) {
@@ -73,6 +74,7 @@ void cut(pa_plan& plan, int tile, const int32_t* lens, int batch, int hkv, int r
     plan.cta_seg_begin.assign(1, 0);
     if (total == 0) return;
     const long per = (total + requested - 1) / requested;
+    plan.per      = static_cast<int>(std::min<long>(per, INT_MAX));
     plan.num_ctas = static_cast<int>((total + per - 1) / per);
     plan.cta_seg_begin.resize(static_cast<size_t>(plan.num_ctas) + 1);
     // Every unit boundary adds at most one segment to the items' own.
@@ -165,6 +167,31 @@ pa_split_shape split_shape(const pa_plan& plan) {
     }
     return sh;
 }
+// Tiles per unit of a plan that cuts its items, whole and in order, into equal
+// ranges of tiles (the last unit may hold fewer), as make_plan does; 0 for others.
+int equal_cut(const pa_plan& plan) {
+    auto tiles = [&](int sg) {
+        const int32_t* s = &plan.segments[4 * static_cast<size_t>(sg)];
+        return (s[3] - s[2] + plan.tile - 1) / plan.tile;
+    };
+    long per = 0;
+    for (int u = 0; u < plan.num_ctas; ++u) {
+        long n = 0;
+        for (int sg = plan.cta_seg_begin[u]; sg < plan.cta_seg_begin[u + 1]; ++sg) n += tiles(sg);
+        if (u == 0) per = n;
+        if (n <= 0 || n > per || (n < per && u + 1 < plan.num_ctas)) return 0;
+    }
+    for (int i = 0; i < plan.items; ++i) {
+        int at = 0;
+        for (int sg = plan.item_seg_begin[i]; sg < plan.item_seg_begin[i + 1]; ++sg) {
+            const int32_t* s = &plan.segments[4 * static_cast<size_t>(sg)];
+            const bool last = sg + 1 == plan.item_seg_begin[i + 1];
+            if (s[2] != at || (!last && s[3] % plan.tile != 0)) return 0;
+            at = s[3];
+        }
+    }
+    return static_cast<int>(std::min<long>(per, INT_MAX));
+}
 // The split kernel's combine of a spanning item runs on one CU and reads one
 // partial per block. Up to 8 blocks per item that is as fast as a merge launch
 // or faster; past 8 the split kernel leaves one partial per block and the merge
@@ -200,6 +227,116 @@ void make_plan_impl(pa_plan& plan, int dtype, const int32_t* lens, int batch, in
     if (num_ctas <= 0) num_ctas = wave_ctas_impl(dtype, hd, group);
     cut(plan, tile, lens, batch, hkv, num_ctas);
 }
+
+namespace {
+// Time a block takes per tile (8 KiB of K and V) with `blocks` of them running,
+// in us: one CU alone streams 67 GB/s, 256 together 27 GB/s each, and between
+// the two the measured time is linear (rows of 500 tokens, fp16, one block per
+// (row, kv head): 8 blocks 67 GB/s per CU, 32 52, 128 36).
+double tile_us(double blocks) { return 0.122 + 0.00071 * blocks; }
+// What merging across blocks adds after a block's last wave, in us: the partial
+// row stored, the arrival, the combine (FP8's blocks hold more rows).
+constexpr double kSpanUs16 = 1.6, kSpanUs32 = 2.4;   // fp16, FP8 (16- and 32-token tiles)
+
+// make_plan's equal cut leaves most items across two or more blocks unless their
+// tiles happen to be whole blocks. Where that costs more than uneven blocks do,
+// the plan runs cut again so that no item spans blocks: every block takes whole
+// items (one each where there are no more items than blocks, else runs of them
+// with the smallest largest block), in equal ranges over its units. The
+// estimates of both: the plan's blocks are equal; uneven ones run together for
+// the average block and the rest of the largest at less than half of them.
+// Same box, us per step, across blocks -> inside: fp16 1 x 200 7.0 -> 5.4, 32 x
+// 200 10.0 -> 7.2, 32 x 1000 24.7 -> 22.3, 32 x 5000 102 -> 97, 128 rows of 100
+// to 200 17.9 -> 16.4; FP8 16 x 200 8.0 -> 5.7, 32 x 2000 25.5 -> 23.0. Left
+// across blocks by the estimate, fp16: 1 x 500 6.9 (8.0 inside), 16 x 500 10.1
+// (11.1), 32 rows of 300 to 1000 17.1 (19.0). Only for the plan that make_plan
+// gives a grid of its own choice (`units`), whoever brings it: another grid is
+// the caller's. The host plan stays as it is. False: not cut.
+bool cut_in_blocks(const pa_plan& plan, int units, pa_plan& out) {
+    const int items = plan.items, max_blocks = units / pa::kBlockUnits;
+    if (items <= 0 || max_blocks <= 0 || plan.per <= 0) return false;
+    std::vector<int32_t> tiles(static_cast<size_t>(items));
+    int  longest = 0;
+    long total   = 0;
+    for (int i = 0; i < items; ++i) {
+        const int len = plan.segments[4 * static_cast<size_t>(plan.item_seg_begin[i + 1]) - 1];
+        tiles[static_cast<size_t>(i)] = (len + plan.tile - 1) / plan.tile;
+        longest = std::max(longest, tiles[static_cast<size_t>(i)]);
+        total += tiles[static_cast<size_t>(i)];
+    }
+    if (plan.per != (total + units - 1) / units) return false;
+    const double across = static_cast<double>(pa::kBlockUnits) * plan.per * tile_us(plan.num_ctas / 8.0) +
+                          (plan.tile == 16 ? kSpanUs16 : kSpanUs32);
+    auto inside = [&](long largest, int blocks) {
+        const double mean = static_cast<double>(total) / blocks;
+        return mean * tile_us(blocks) + (static_cast<double>(largest) - mean) * tile_us(0.4 * blocks);
+    };
+    const bool one_each = items <= max_blocks;
+    long cap = longest;
+    if (one_each) {
+        if (inside(longest, items) >= across) return false;
+    } else {
+        // The smallest cap, to 1/32, under which greedy runs need no more blocks.
+        cap = std::max<long>(cap, (total + max_blocks - 1) / max_blocks);
+        for (;; cap += cap / 32 + 1) {
+            if (inside(cap, max_blocks) >= across) return false;
+            int  blocks = 0;
+            long left   = 0;
+            for (const int32_t t : tiles) {
+                if (t > left) ++blocks, left = cap;
+                left -= t;
+            }
+            if (blocks <= max_blocks) break;
+        }
+    }
+    out.num_ctas = 0;
+    out.tile     = plan.tile;
+    out.items    = items;
+    out.shape    = {};
+    out.segments.clear();
+    out.cta_seg_begin.clear();
+    out.segments.reserve(plan.segments.size());
+    out.item_seg_begin.resize(static_cast<size_t>(items) + 1);
+    for (int i = 0; i < items;) {
+        int  end  = i + 1;
+        long load = tiles[static_cast<size_t>(i)];
+        while (!one_each && end < items && load + tiles[static_cast<size_t>(end)] <= cap)
+            load += tiles[static_cast<size_t>(end++)];
+        const long per = (load + pa::kBlockUnits - 1) / pa::kBlockUnits;
+        long left = per;
+        out.cta_seg_begin.push_back(static_cast<int32_t>(out.segments.size() / 4));
+        for (; i < end; ++i) {
+            const size_t  last  = 4 * static_cast<size_t>(plan.item_seg_begin[i + 1]) - 4;   // the item's last segment
+            const int     row = plan.segments[last], head = plan.segments[last + 1], len = plan.segments[last + 3];
+            const int32_t first = static_cast<int32_t>(out.segments.size() / 4);
+            out.item_seg_begin[static_cast<size_t>(i)] = first;
+            for (long done = 0; done < tiles[static_cast<size_t>(i)];) {
+                if (left == 0) {
+                    out.cta_seg_begin.push_back(static_cast<int32_t>(out.segments.size() / 4));
+                    left = per;
+                }
+                const long take = std::min<long>(left, tiles[static_cast<size_t>(i)] - done);
+                out.segments.insert(out.segments.end(),
+                                    {row, head, static_cast<int32_t>(done * plan.tile),
+                                     static_cast<int32_t>(std::min<long>((done + take) * plan.tile, len))});
+                done += take;
+                left -= take;
+            }
+            const int n = static_cast<int>(out.segments.size() / 4) - first;
+            out.shape.max_segments = std::max(out.shape.max_segments, n);
+            if (n > 1) out.shape.split = true, out.shape.max_blocks = 1;
+        }
+        // The block's unused units are empty.
+        out.num_ctas += pa::kBlockUnits;
+        out.cta_seg_begin.resize(static_cast<size_t>(out.num_ctas), static_cast<int32_t>(out.segments.size() / 4));
+    }
+    const int32_t nseg = static_cast<int32_t>(out.segments.size() / 4);
+    out.item_seg_begin[static_cast<size_t>(items)] = nseg;
+    out.cta_seg_begin.push_back(nseg);
+    // The workspace (used if a caller forces the merge kernel) holds the plan's count.
+    return out.segments.size() <= plan.segments.size();
+}
+}  // namespace
 namespace {
 // Whether the copy kernel of the buffer's last use has read it.
 bool stage_read(const pa_stage& st) {
@@ -298,15 +435,20 @@ void device_plan_upload(pa_device_plan& dp, const pa_plan& plan, int group, int 
     for (size_t i = 0; i < nseg; ++i)
         if (plan.segments[4 * i + 2] % pa::kGroupTokens != 0)
             throw std::invalid_argument("upload: segment starts must be multiples of 16 tokens");
+    const bool kernel_tile = plan.tile == pa::kernel_tile_tokens(PA_KV_FP16, group) ||
+                             plan.tile == pa::kernel_tile_tokens(PA_KV_FP8_E4M3, group);
+    const bool snap = kernel_tile && plan.per > 0 && plan_merge_mode(plan) == 2 &&
+                      cut_in_blocks(plan, device_cus() * pa::kernel_units_per_cu(PA_KV_FP16, group), dp.blocks);
+    const pa_plan& run = snap ? dp.blocks : plan;   // what the device gets
     // One block: segments | cta_seg_begin | item_seg_begin | extra | merge
     // counters, each part starting on a 16-byte boundary (the kernels read
     // segments as int4).
     auto round4 = [](size_t n) { return (n + 3) & ~size_t{3}; };
-    const size_t o_cta   = round4(plan.segments.size());
-    const size_t o_item  = o_cta + round4(plan.cta_seg_begin.size());
-    const size_t o_extra = o_item + round4(plan.item_seg_begin.size());
+    const size_t o_cta   = round4(run.segments.size());
+    const size_t o_item  = o_cta + round4(run.cta_seg_begin.size());
+    const size_t o_extra = o_item + round4(run.item_seg_begin.size());
     const size_t o_ctr   = o_extra + round4(n_extra);   // per-item merge counters, uploaded as zeros
-    const pa_split_shape& shape = plan.shape;
+    const pa_split_shape& shape = run.shape;
     const int  in_kernel = merge_mode_of(shape, kChainMaxBlocks);
     // Past kChainMaxBlocks: block partials for the merge kernel (block_merge 3),
     // where the split kernel can find an item's part of a block. Same box, us per
@@ -330,9 +472,9 @@ void device_plan_upload(pa_device_plan& dp, const pa_plan& plan, int group, int 
         dp.ints_cap = cap;
     }
     pa_stage& st = take_stage(dp.staging, total, false);
-    std::copy(plan.segments.begin(), plan.segments.end(), st.host);
-    std::copy(plan.cta_seg_begin.begin(), plan.cta_seg_begin.end(), st.host + o_cta);
-    std::copy(plan.item_seg_begin.begin(), plan.item_seg_begin.end(), st.host + o_item);
+    std::copy(run.segments.begin(), run.segments.end(), st.host);
+    std::copy(run.cta_seg_begin.begin(), run.cta_seg_begin.end(), st.host + o_cta);
+    std::copy(run.item_seg_begin.begin(), run.item_seg_begin.end(), st.host + o_item);
     if (n_extra) std::copy(extra, extra + n_extra, st.host + o_extra);
     std::fill(st.host + o_ctr, st.host + o_unit, 0);
     if (blocks) std::copy(shape.item_unit.begin(), shape.item_unit.end(), st.host + o_unit);
@@ -352,7 +494,7 @@ void device_plan_upload(pa_device_plan& dp, const pa_plan& plan, int group, int 
         dp.part_cap = need;
     }
     dp.partial_lse = dp.partial_out ? dp.partial_out + rows * head_dim : nullptr;
-    dp.num_ctas = plan.num_ctas;
+    dp.num_ctas = run.num_ctas;
     dp.num_segments = static_cast<int>(nseg);
     dp.block_merge = blocks ? 3 : in_kernel;
     dp.needs_merge = blocks || (in_kernel == 0 && shape.split) ? 1 : 0;
@@ -487,6 +629,7 @@ pa_status pa_plan_create(int num_ctas, int tile, const int32_t* segments, int nu
         plan->cta_seg_begin.assign(cta_seg_begin, cta_seg_begin + num_ctas + 1);
         plan->item_seg_begin.assign(item_seg_begin, item_seg_begin + num_items + 1);
         plan->shape    = split_shape(*plan);
+        plan->per      = equal_cut(*plan);
         *out = plan;
     });
 }

@@ -83,7 +83,7 @@ def stamps_of(s: Setup, steps: int = 200, flusher: Flusher | None = None) -> dic
             b.synchronize()
             ms.append(a.elapsed_time(b))
         period_ms = sorted(ms)[len(ms) // 2]
-    nb = (s.plan.num_ctas + 7) // 8
+    nb = (s.params.num_ctas + 7) // 8   # the device plan's grid
     buf = np.zeros(nb * SLOTS, np.uint64)
     if lib.pa_debug_stamps(buf.ctypes.data, buf.nbytes) != 0:
         raise RuntimeError("pa_debug_stamps failed")

@@ -69,12 +69,71 @@ def test_many_split_rows_in_a_block(fp8, group):
     _check(fp8, lens, group, 8, plan.handle.value, 2)
 
 
-@pytest.mark.parametrize("lens,ctas", [([100], 0), ([129], 0), ([16 * 17] * 3, 0), ([5000, 1, 700, 16, 17], 96)],
-                         ids=["7_tiles", "9_tiles", "17_tiles", "mixed"])
+@pytest.mark.parametrize("lens,ctas", [([100], 28), ([129], 36), ([16 * 17] * 3, 204), ([528], 0),
+                                       ([5000, 1, 700, 16, 17], 96)],
+                         ids=["7_tiles", "9_tiles", "17_tiles", "33_tiles", "mixed"])
 def test_short_rows_across_blocks(lens, ctas):
     """Rows that straddle two or three blocks because their tiles are no multiple of a block's units."""
     plan = _plan(False, lens, 4, 8, ctas)
     _check(False, lens, 4, 8, plan.handle.value, 2)
+
+
+def _device_plan_arrays(p, items):
+    from helpers import d2h
+    cta = d2h(int(p.cta_seg_begin), 4 * (p.num_ctas + 1), np.int32)
+    item = d2h(int(p.item_seg_begin), 4 * (items + 1), np.int32)
+    return cta, item, d2h(int(p.segments), 16 * int(cta[-1]), np.int32).reshape(-1, 4)
+
+
+@pytest.mark.parametrize("lens,fp8,group,hkv", [
+    ([200], False, 4, 8),                          # one item per block, fewer blocks than the chip has
+    ([33], False, 2, 8),                           # three tiles per item
+    ([200] * 32, False, 4, 8),                     # as many items as blocks
+    ([1100] * 32, True, 8, 8),
+    ([10, 33, 300, 1, 64, 250, 17, 129], True, 1, 8),
+    ([100, 150, 200, 130, 170, 110, 190, 120] * 16, False, 4, 8),   # several items per block
+    ([1, 9, 33, 20, 16, 31, 2, 40, 17] * 6, False, 8, 8),           # many short items per block
+    ([95, 161, 128] * 40, True, 4, 4),
+], ids=["row", "three_tiles", "full", "g8", "ragged", "packed", "short", "fp8_packed"])
+def test_items_kept_inside_blocks(lens, fp8, group, hkv):
+    """Plans of make_plan's own grid whose items would straddle blocks run cut again: every block of 8 units
+    holds whole items, every token once and in order, and the decode matches the oracle and the merge kernel."""
+    plan = _plan(fp8, lens, group, hkv, 0)
+    assert plan.merge_mode == 2
+    dplan = pa_amd.DevicePlan()
+    dplan.upload(plan, group, D)
+    p = pa_amd.DecodeParams()
+    dplan.bind(p)
+    assert p.block_merge == 1 and p.num_segments == len(plan.segments) and p.num_ctas % 8 == 0
+    cta, item, seg = _device_plan_arrays(p, len(lens) * hkv)
+    assert len(seg) <= len(plan.segments) and np.all(np.diff(cta) >= 0) and item[-1] == len(seg)
+    unit = np.repeat(np.arange(p.num_ctas), np.diff(cta))
+    for i in range(len(lens) * hkv):
+        rows = seg[item[i]:item[i + 1]]
+        assert len(rows) and np.all(rows[:, 0] == i // hkv) and np.all(rows[:, 1] == i % hkv)
+        assert rows[0, 2] == 0 and rows[-1, 3] == lens[i // hkv] and np.array_equal(rows[1:, 2], rows[:-1, 3])
+        u = unit[item[i]:item[i + 1]]
+        assert u[0] // 8 == u[-1] // 8 and np.array_equal(u, np.arange(u[0], u[0] + len(u)))
+    for u in range(p.num_ctas):     # a unit's split segments are its first and last
+        split = [s for s in range(cta[u], cta[u + 1]) if np.sum(unit[item[seg[s, 0] * hkv + seg[s, 1]]:
+                                                                   item[seg[s, 0] * hkv + seg[s, 1] + 1]] >= 0) > 1]
+        assert all(s in (cta[u], cta[u + 1] - 1) for s in split)
+    _check(fp8, lens, group, hkv, plan.handle.value, 1, repeats=2)
+
+
+def test_another_grid_is_left_as_it_is():
+    """A caller's grid, and rows that are cheaper across blocks, keep the host plan's arrays."""
+    for lens, ctas in (([200] * 32, 512), ([500], 0), ([300, 1000, 450, 700] * 8, 0)):
+        plan = _plan(False, lens, 4, 8, ctas)
+        assert plan.merge_mode == 2
+        dplan = pa_amd.DevicePlan()
+        dplan.upload(plan, 4, D)
+        p = pa_amd.DecodeParams()
+        dplan.bind(p)
+        assert p.block_merge == 2 and p.num_ctas == plan.num_ctas
+        cta, item, seg = _device_plan_arrays(p, len(lens) * 8)
+        assert np.array_equal(seg, plan.segments) and np.array_equal(cta, plan.cta_seg_begin)
+        assert np.array_equal(item, plan.item_seg_begin)
 
 
 @pytest.mark.parametrize("group", [1, 4, 8])
