@@ -86,18 +86,18 @@ typedef struct pa_decode_params {
                                           block of 8 work units and is merged there in LDS.
                                           2: items spanning blocks are also merged in the
                                           split kernel: each block writes one partial per
-                                          such item to the workspace, and the last block
-                                          to finish (merge_counters) combines them.
+                                          such item to the workspace, and the last to
+                                          finish (merge_counters) combines them.
                                           3: each block writes such partials as under 2 and
                                           the merge kernel combines them (items over more
                                           blocks than 2 takes). */
     int32_t         num_segments;      /* segments of the bound plan (0 = unknown); sizes the
                                           partial workspace. Set by bind. */
-    int32_t*        merge_counters;    /* block_merge 2: one arrival counter per item, zero
-                                          between decodes (the plan zeroes them at upload;
-                                          every decode leaves them at zero). block_merge 3:
-                                          each item's first work unit follows them. Set by
-                                          bind. */
+    int32_t*        merge_counters;    /* block_merge 2: arrival counters (one per item and 256
+                                          of its group x head_dim outputs), zero between
+                                          decodes (the plan zeroes them at upload; every decode
+                                          leaves them at zero). block_merge 3: each item's
+                                          first work unit follows them. Set by bind. */
 } pa_decode_params;
 
 /* Thread-local message describing the last failed call ("" if none). */

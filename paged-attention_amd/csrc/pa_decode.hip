@@ -60,8 +60,8 @@
 //     (tasks of 256 elements of one row). A row inside the block (e.g. 32 rows x 8 kv heads x
 //     8192 tokens over 2048 units) is then complete; a row that spans blocks
 //     (up to 8) leaves one device-coherent partial per block, and the last
-//     of its blocks to arrive (a per-row counter) combines them, in block
-//     order. No merge launch is needed. Where a row spans more blocks
+//     wave to arrive (a counter per row and 256 elements) combines them, in
+//     block order. No merge launch is needed. Where a row spans more blocks
 //     (block_merge 3) each block leaves such a partial for the merge kernel.
 //     Otherwise (caller plans that do not keep a row's segments in consecutive
 //     units, and rows of one query head over fewer than 64 blocks) every split
@@ -338,126 +338,6 @@ struct alignas(16) Slot {
     int item, seg, s0, n;
 };
 
-// An item of this block that spans blocks.
-struct Span {
-    int item, s0, n, u0;   // u0: the unit of its first segment
-};
-
-// The last block of a spanning item combines the item's block partials (block
-// j's sits at the item's first segment in block j). They are summed in NGR
-// states per 16-byte dim vector, state g taking every NGR-th block from g on,
-// each with one coherent 16-byte load of the row and one of its LSE, all issued
-// before the first is used (one round trip), with a running maximum in block
-// order; the states of a vector then meet in a fixed tree (1, 2, 4, 8 apart).
-// A block that is last for one item has one state per thread; a block that is
-// last for two has S = 2 states per thread and half its threads on each item,
-// side by side. The tree's sums are rounded the same from both sides
-// (no contraction), so the result depends neither on S nor on timing.
-template <int G, int S>
-__device__ __forceinline__ void combine_blocks(const pa_decode_params& p, const Span& it, int t) {
-#pragma clang fp contract(off)
-    constexpr int NO  = G * kHeadDim;
-    constexpr int NV  = NO / 4;                   // 16-byte vectors of one block partial
-    constexpr int NGR = 64 * kWaves / NV;         // states of one vector (16, 8, 4, 2 for G = 1, 2, 4, 8)
-    constexpr int LPV = NGR / S;                  // lanes sharing one vector
-    constexpr int U   = NGR >= 8 ? 1 : 8 / NGR;   // loads per state and round (8 blocks)
-    static_assert(S == 1 || S == 2, "one or two states per thread");
-    static_assert(LPV >= 1 && LPV <= 16 && (LPV & (LPV - 1)) == 0, "the lanes of a vector lie in one DPP row");
-    const int li = t % LPV;
-    const int vi = t / LPV;
-    const int hh = 4 * vi / kHeadDim;            // query head of the vector
-    const int j0 = it.u0 / kWaves, j1 = (it.u0 + it.n - 1) / kWaves;
-    // The item's partial rows and LSEs, from its first segment on (byte
-    // offsets fit 32 bits: n segments of NO floats).
-    const __amdgpu_buffer_rsrc_t rs =
-        buffer_rsrc(p.partial_out + static_cast<size_t>(it.s0) * NO, it.n * NO * static_cast<int>(sizeof(float)));
-    const __amdgpu_buffer_rsrc_t rl =
-        buffer_rsrc(p.partial_lse + static_cast<size_t>(it.s0) * G, it.n * G * static_cast<int>(sizeof(float)));
-    float m[S], den[S];
-    f32x4 acc[S];
-#pragma unroll
-    for (int s = 0; s < S; ++s) {
-        m[s]   = -INFINITY;
-        den[s] = 0.f;
-        acc[s] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-    for (int jb = j0; jb <= j1; jb += NGR * U) {
-        u32x4 raw[S][U];
-        float ls[S][U];
-#pragma unroll
-        for (int s = 0; s < S; ++s)
-#pragma unroll
-            for (int k = 0; k < U; ++k) {
-                const int j = jb + S * li + s + NGR * k;
-                if (j <= j1) {
-                    const int sg = max(0, kWaves * j - it.u0);   // the block's first segment, from s0
-                    raw[s][k] = __builtin_bit_cast(
-                        u32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                   rs, (sg * NO + 4 * vi) * static_cast<int>(sizeof(float)), 0, kAuxCoherent));
-                    ls[s][k] = __builtin_bit_cast(
-                        float, __builtin_amdgcn_raw_buffer_load_b32(
-                                   rl, (sg * G + hh) * static_cast<int>(sizeof(float)), 0, kAuxCoherent));
-                }
-            }
-#if PA_STAMPS
-        __builtin_amdgcn_s_waitcnt(kWaitVm0);
-        if (t == 0 && jb == j0) stamp(12);
-#endif
-#pragma unroll
-        for (int s = 0; s < S; ++s)
-#pragma unroll
-            for (int k = 0; k < U; ++k) {
-                if (jb + S * li + s + NGR * k > j1) break;
-                const float mn  = fmaxf(m[s], ls[s][k]);
-                const float f   = exp2_fast(m[s] - mn);   // 0 while m = -inf
-                const float wgt = exp2_fast(ls[s][k] - mn);
-                const f32x4 v   = __builtin_bit_cast(f32x4, raw[s][k]);
-#pragma unroll
-                for (int c = 0; c < 4; ++c) acc[s][c] = fmaf(wgt, v[c], acc[s][c] * f);
-                den[s] = fmaf(den[s], f, wgt);
-                m[s]   = mn;
-            }
-    }
-    // The tree (a state with no block has m = -inf and weighs 0).
-    auto combine = [&](float m2, float d2, const f32x4& a2) {
-        const float mt = fmaxf(m[0], m2);
-        const float f1 = m[0] == -INFINITY ? 0.f : exp2_fast(m[0] - mt);
-        const float f2 = m2 == -INFINITY ? 0.f : exp2_fast(m2 - mt);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) acc[0][c] = acc[0][c] * f1 + a2[c] * f2;
-        den[0] = den[0] * f1 + d2 * f2;
-        m[0]   = mt;
-    };
-    auto partner_round = [&](auto ctrl) {
-        constexpr int C = decltype(ctrl)::value;
-        f32x4 a2;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) a2[c] = dpp_f32<C>(acc[0][c]);
-        combine(dpp_f32<C>(m[0]), dpp_f32<C>(den[0]), a2);
-    };
-    if (t == 0) stamp(13);
-    // A round whose partners hold no block changes nothing and is left out.
-    const int nb = j1 - j0 + 1;
-    if constexpr (S == 2) combine(m[1], den[1], acc[1]);
-    if constexpr (LPV >= 2)
-        if (nb > S) partner_round(std::integral_constant<int, 0xB1>{});        // quad_perm [1,0,3,2]
-    if constexpr (LPV >= 4)
-        if (nb > 2 * S) partner_round(std::integral_constant<int, 0x4E>{});    // quad_perm [2,3,0,1]
-    if constexpr (LPV >= 8)
-        if (nb > 4 * S) partner_round(std::integral_constant<int, 0x141>{});   // row_half_mirror
-    if constexpr (LPV >= 16)
-        if (nb > 8 * S) partner_round(std::integral_constant<int, 0x140>{});   // row_mirror
-    if (t == 0) stamp(14);
-    if (li == 0) {
-        const float inv = 1.0f / den[0];
-        const f16x2 lo = {static_cast<_Float16>(acc[0][0] * inv), static_cast<_Float16>(acc[0][1] * inv)};
-        const f16x2 hi = {static_cast<_Float16>(acc[0][2] * inv), static_cast<_Float16>(acc[0][3] * inv)};
-        *reinterpret_cast<u32x2*>(p.out + static_cast<size_t>(it.item) * NO + 4 * vi) =
-            u32x2{__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi)};
-    }
-    if (t == 0) stamp(15);
-}
-
 // Block-level merge after the split loop. `slots` holds, per wave, its first
 // (slot 0) and last (slot 1) segment when that segment is a split one; part /
 // lse hold the slot's normalized partial rows and base-2 LSEs, written to LDS
@@ -485,19 +365,24 @@ __device__ __forceinline__ void combine_blocks(const pa_decode_params& p, const 
 // block at the block's first slot and into the next at its last): the block's
 // average becomes one partial row of the item, at the workspace slot of the
 // item's first segment in the block, with LSE max + log2(sum of weights).
-// Under block_merge 3 the merge kernel does the rest. Under 2,
-// after every thread's stores are complete, one lane per such item adds one to
-// the item's counter; the block that brings it to the item's block count
-// resets it to zero and combines the item's block partials, in block order, as
-// the merge kernel does (so the result does not depend on which block is
-// last). Blocks never wait for each other.
+// Under block_merge 3 the merge kernel does the rest. Under 2 the tasks meet
+// across blocks one by one: a wave waits for its own stores, adds one to the
+// counter of (item, task), and the wave that brings it to the item's block count
+// resets it to zero and combines the item's block partials of its 256 elements
+// in block order (so the result does not depend on which block is last).
+// Blocks never wait for each other, and no barrier lies between a task's store,
+// arrival and combine. (With the block's waves arriving together, behind a
+// barrier, and the last block combining with all of them behind another: 4 x
+// 1024 9.0 us per step against 8.6, 32 x 8192 over one kv head 25.3 / 24.7, 32
+// rows of 64 to 1000 14.7 / 14.1, 12 rows to 9000 with 64 query heads 32.8 / 32.1.)
 template <int G>
 __device__ __forceinline__ void block_merge(const pa_decode_params& p, const Slot* slots,
                                             const float (*part)[G * kHeadDim], const float (*lse)[G],
-                                            int* last_lds, int tid, int lblock) {
+                                            int tid, int lblock) {
     constexpr int NS  = 2 * kWaves;
     constexpr int NO  = G * kHeadDim;
-    constexpr int TPR = NO > 256 ? NO / 256 : 1;   // tasks per run
+    constexpr int TPR = merge_tasks(G);   // tasks per run
+    static_assert(TPR == (NO > 256 ? NO / 256 : 1), "tasks of 256 elements");
     static_assert(NS == 16, "the slots fit the low lanes of a wave");
     const int  lane  = tid & 63;
     const int  wave  = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -517,114 +402,139 @@ __device__ __forceinline__ void block_merge(const pa_decode_params& p, const Slo
         const uint32_t upto = next ? (next & (0u - next)) - 1u : ~0u;   // the slots before it
         return filled & upto & ~((from & (0u - from)) - 1u);
     };
-    const int runs = __builtin_popcount(starts);
+    const int runs  = __builtin_popcount(starts);
+    const int items = p.batch * p.num_kv_heads;
     for (int t = wave; t < runs * TPR; t += kWaves) {
-        uint32_t from = starts;
-        for (int r = t / TPR; r > 0; --r) from &= from - 1;
+        // The block's first and last run, which may span, come first.
+        const int r = t / TPR;
+        uint32_t from = r == 1 ? 1u << (31 - __builtin_clz(starts)) : starts;
+        for (int k = r; k > 1; --k) from &= from - 1;
         const uint32_t run  = run_of(from);
         const int  j0    = __builtin_ctz(from);
         const int  item  = __builtin_amdgcn_readlane(mine.item, j0);
         const int  bseg  = __builtin_amdgcn_readlane(mine.seg, j0);   // the item's first segment here
+        const int  s0    = __builtin_amdgcn_readlane(mine.s0, j0);
         const int  n     = __builtin_amdgcn_readlane(mine.n, j0);
         const bool spans = chain && __builtin_popcount(run) != n;
 #if PA_STAMPS
         if (tid == 0 && t == 0) stamp(18 + spans);
 #endif
-        const int o = 256 * (t % TPR) + 4 * lane;
-        if (NO >= 256 || o < NO) {
-            const int hd = o / kHeadDim;
-            float mx = -INFINITY, den = 0.f;
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-            // Eight slots at a time (every plan of make_plan's has at most
-            // eight in a run): all their LDS reads, then the weights. Past
-            // the run's end nothing is read and the weight is 0.
-            for (uint32_t rem = run; rem != 0;) {
-                float ls[8];
-                f32x4 v[8];
+        const int  o    = 256 * (t % TPR) + 4 * lane;
+        const bool live = NO >= 256 || o < NO;
+        const int  hd   = live ? o / kHeadDim : 0;
+        float mx = -INFINITY, den = 0.f;
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        // Adds eight partials with their LSEs (-inf: none, weight 0).
+        auto add8 = [&](const float (&ls)[8], const f32x4 (&v)[8]) {
+            float mn = mx;
 #pragma unroll
-                for (int k = 0; k < 8; ++k) {
-                    ls[k] = -INFINITY;
-                    v[k]  = f32x4{0.f, 0.f, 0.f, 0.f};
-                    if (rem) {
-                        const int j = __builtin_ctz(rem);
-                        rem &= rem - 1;
-                        ls[k] = lse[j][hd];
-                        v[k]  = *reinterpret_cast<const f32x4*>(&part[j][o]);
-                    }
-                }
-                float mn = mx;
+            for (int k = 0; k < 8; ++k) mn = fmaxf(mn, ls[k]);
+            const float f = exp2_fast(mx - mn);   // 0 at the first eight
+            den *= f;
 #pragma unroll
-                for (int k = 0; k < 8; ++k) mn = fmaxf(mn, ls[k]);
-                const float f = exp2_fast(mx - mn);   // 0 at the first eight
-                den *= f;
+            for (int c = 0; c < 4; ++c) acc[c] *= f;
 #pragma unroll
-                for (int c = 0; c < 4; ++c) acc[c] *= f;
+            for (int k = 0; k < 8; ++k) {
+                const float w = exp2_fast(ls[k] - mn);
 #pragma unroll
-                for (int k = 0; k < 8; ++k) {
-                    const float w = exp2_fast(ls[k] - mn);
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) acc[c] = fmaf(w, v[k][c], acc[c]);
-                    den += w;
-                }
-                mx = mn;
+                for (int c = 0; c < 4; ++c) acc[c] = fmaf(w, v[k][c], acc[c]);
+                den += w;
             }
+            mx = mn;
+        };
+        auto write_out = [&]() {
             const float inv = 1.0f / den;
-            if (!spans) {
-                const f16x2 lo = {static_cast<_Float16>(acc[0] * inv), static_cast<_Float16>(acc[1] * inv)};
-                const f16x2 hi = {static_cast<_Float16>(acc[2] * inv), static_cast<_Float16>(acc[3] * inv)};
+            const f16x2 lo = {static_cast<_Float16>(acc[0] * inv), static_cast<_Float16>(acc[1] * inv)};
+            const f16x2 hi = {static_cast<_Float16>(acc[2] * inv), static_cast<_Float16>(acc[3] * inv)};
+            if (live)
                 *reinterpret_cast<u32x2*>(p.out + static_cast<size_t>(item) * NO + o) =
                     u32x2{__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi)};
-            } else {
-                const __amdgpu_buffer_rsrc_t rs = buffer_rsrc(p.partial_out + static_cast<size_t>(bseg) * NO,
-                                                              NO * static_cast<int>(sizeof(float)));
-                store_coherent16(rs, o * static_cast<int>(sizeof(float)),
-                                 f32x4{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv});
-                if (o % kHeadDim == 0)
-                    store_coherent(p.partial_lse + static_cast<size_t>(bseg) * G + hd, mx + __log2f(den));
+        };
+        // Eight slots at a time (every plan of make_plan's has at most eight in
+        // a run): all their LDS reads, then the weights. Past the run's end
+        // nothing is read.
+        for (uint32_t rem = run; rem != 0;) {
+            float ls[8];
+            f32x4 v[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                ls[k] = -INFINITY;
+                v[k]  = f32x4{0.f, 0.f, 0.f, 0.f};
+                if (rem) {
+                    const int j = __builtin_ctz(rem);
+                    rem &= rem - 1;
+                    ls[k] = lse[j][hd];
+                    v[k]  = *reinterpret_cast<const f32x4*>(&part[j][live ? o : 0]);
+                }
             }
+            add8(ls, v);
         }
-    }
-    if (p.block_merge != 2) return;   // 3: the merge kernel combines the block partials
-    // Items of this block that span blocks: its first run, its last, or both
-    // (sa; sb when there are two).
-    auto span_of = [&](uint32_t from) {
-        const int j0 = __builtin_ctz(from);
-        const int s0 = __builtin_amdgcn_readlane(mine.s0, j0);
-        const int u0 = lblock * kWaves + (j0 >> 1) - (__builtin_amdgcn_readlane(mine.seg, j0) - s0);
-        return Span{__builtin_amdgcn_readlane(mine.item, j0), s0, __builtin_amdgcn_readlane(mine.n, j0), u0};
-    };
-    const uint32_t last_start = 1u << (31 - __builtin_clz(starts));
-    const Span     first_run  = span_of(starts), last_run = span_of(last_start);
-    const bool     first_spans = __builtin_popcount(run_of(starts)) != first_run.n;
-    const bool     last_spans  = runs > 1 && __builtin_popcount(run_of(last_start)) != last_run.n;
-    if (!first_spans && !last_spans) return;
-    const int  ns = first_spans && last_spans ? 2 : 1;
-    const Span sa = first_spans ? first_run : last_run;
-    const Span sb = last_run;
-    if (tid == 0) stamp(9);
-
-    // Arrivals: this block's partial rows are complete at the coherence point
-    // before its counters move.
-    __builtin_amdgcn_s_waitcnt(kWaitVm0);
-    __syncthreads();
-    if (tid == 0) stamp(10);
-    if (tid < ns) {
-        const Span it = tid == 0 ? sa : sb;
-        const int  nb = (it.u0 + it.n - 1) / kWaves - it.u0 / kWaves + 1;   // blocks the item spans
-        int* ctr = p.merge_counters + it.item;
-        const int before = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const bool last = before == nb - 1;
-        if (last) __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // for the next decode
-        last_lds[tid] = last;
-    }
-    __syncthreads();
-    if (tid == 0) stamp(11);
-    const bool last_a = last_lds[0] != 0, last_b = ns > 1 && last_lds[1] != 0;
-    if (last_a && last_b) {
-        const bool lower = wave < kWaves / 2;
-        combine_blocks<G, 2>(p, lower ? sa : sb, lower ? tid : tid - 32 * kWaves);
-    } else if (last_a || last_b) {
-        combine_blocks<G, 1>(p, last_a ? sa : sb, tid);
+        if (!spans) {
+            write_out();
+            continue;
+        }
+        // The item's partial rows and LSEs, from its first segment on (byte
+        // offsets fit 32 bits: n segments of NO floats).
+        const __amdgpu_buffer_rsrc_t rs =
+            buffer_rsrc(p.partial_out + static_cast<size_t>(s0) * NO, n * NO * static_cast<int>(sizeof(float)));
+        const __amdgpu_buffer_rsrc_t rl =
+            buffer_rsrc(p.partial_lse + static_cast<size_t>(s0) * G, n * G * static_cast<int>(sizeof(float)));
+        if (live) {
+            const float inv = 1.0f / den;
+            store_coherent16(rs, ((bseg - s0) * NO + o) * static_cast<int>(sizeof(float)),
+                             f32x4{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv});
+            if (o % kHeadDim == 0)
+                store_coherent(p.partial_lse + static_cast<size_t>(bseg) * G + hd, mx + __log2f(den));
+        }
+        if (p.block_merge != 2) continue;   // 3: the merge kernel combines the block partials
+        if (tid == 0) stamp(9);
+        // The wave's stores are complete at the coherence point before its
+        // arrival; what it reads afterwards it reads after the arrival (the
+        // empty asm keeps the compiler from moving either across).
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(kWaitVm0);
+        asm volatile("" ::: "memory");
+        if (tid == 0) stamp(10);
+        const int u0 = lblock * kWaves + (j0 >> 1) - (bseg - s0);   // unit of the item's first segment
+        const int b0 = u0 / kWaves, nb = (u0 + n - 1) / kWaves - b0 + 1;   // blocks it spans
+        int* ctr = p.merge_counters + static_cast<size_t>(t % TPR) * items + item;
+        int before = 0;
+        if (lane == 0) before = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        before = __builtin_amdgcn_readfirstlane(before);
+        if (tid == 0) stamp(11);
+        if (before != nb - 1) continue;
+        asm volatile("" ::: "memory");
+        if (lane == 0) __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // for the next decode
+        mx  = -INFINITY;
+        den = 0.f;
+        acc = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int k0 = 0; k0 < nb; k0 += 8) {
+            float ls[8];
+            f32x4 v[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                ls[k] = -INFINITY;
+                v[k]  = f32x4{0.f, 0.f, 0.f, 0.f};
+                if (k0 + k < nb) {
+                    const int sg = max(0, kWaves * (b0 + k0 + k) - u0);   // the block's first segment, from s0
+                    v[k] = __builtin_bit_cast(
+                        f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                   rs, (sg * NO + (live ? o : 0)) * static_cast<int>(sizeof(float)), 0, kAuxCoherent));
+                    ls[k] = __builtin_bit_cast(
+                        float, __builtin_amdgcn_raw_buffer_load_b32(
+                                   rl, (sg * G + hd) * static_cast<int>(sizeof(float)), 0, kAuxCoherent));
+                }
+            }
+#if PA_STAMPS
+            __builtin_amdgcn_s_waitcnt(kWaitVm0);
+            if (tid == 0 && k0 == 0) stamp(12);
+#endif
+            add8(ls, v);
+        }
+        if (tid == 0) stamp(13);
+        if (tid == 0) stamp(14);
+        write_out();
+        if (tid == 0) stamp(15);
     }
 }
 
@@ -670,7 +580,6 @@ __device__ __forceinline__ void decode_split_body(const pa_decode_params& p, con
     // by issue() with the K / V, 1 KiB per load).
     __shared__ __attribute__((aligned(16))) u32x4 q_lds[kWaves][64 * NQ];
     __shared__ Slot slots[2 * kWaves];                                       // split segments, 2 * wave + sl
-    __shared__ int last_lds[2];                                              // block merges a spanning item
     // LDS stage of one step per wave (STG): [K, V][half][16 rows][row bytes],
     // each row's 16-byte chunks XOR-swizzled by (row % chunks per row).
     __shared__ __attribute__((aligned(16))) u32x4 stage_lds[STG ? kWaves : 1][STG ? 2 * NH * HCH : 1];
@@ -1276,7 +1185,7 @@ __device__ __forceinline__ void decode_split_body(const pa_decode_params& p, con
 
     if (merge_here) {
         __syncthreads();
-        block_merge<G>(p, slots, part_lds, lse_lds, last_lds, threadIdx.x, lblock);
+        block_merge<G>(p, slots, part_lds, lse_lds, threadIdx.x, lblock);
     }
 }
 
@@ -1543,7 +1452,7 @@ hipError_t launch_merge_gd(const pa_decode_params& p, hipStream_t s) {
     constexpr int SPW = 256 / DS;    // segments one wave covers per pass
     const bool blocks = p.block_merge == 3;
     const int  m      = blocks ? (p.max_item_segments + kWaves - 1) / kWaves + 1 : p.max_item_segments;
-    const int32_t* unit0 = blocks ? p.merge_counters + plan_item_units(p.batch * p.num_kv_heads) : nullptr;
+    const int32_t* unit0 = blocks ? p.merge_counters + plan_item_units(p.batch * p.num_kv_heads, G) : nullptr;
     if (m > 0 && m <= 4 * SPW)
         hipLaunchKernelGGL((decode_merge_kernel<G, 1, DS>), grid, dim3(64), 0, s, p.item_seg_begin, p.partial_out,
                            p.partial_lse, p.num_kv_heads, unit0, p);

@@ -81,7 +81,7 @@ struct pa_device_plan {
     int      max_item_segments = 0;
     int      num_segments = 0;
     int      block_merge = 0;          // pa_decode_params.block_merge of the plan
-    int32_t* merge_counters = nullptr;  // per-item counters in `ints`
+    int32_t* merge_counters = nullptr;  // arrival counters in `ints`
     pa_plan  blocks;                    // the plan cut again inside blocks, where that is what runs
     pa_stage_pool staging;
 };

@@ -52,9 +52,14 @@ inline void check_kv_dtype(int dtype) {
         throw std::invalid_argument("unknown kv dtype " + std::to_string(dtype));
 }
 
-// Where a device plan keeps each item's first unit (block_merge 3), in int32
-// elements from its merge counters: after them, on a 16-byte boundary.
-constexpr size_t plan_item_units(int items) { return (static_cast<size_t>(items) + 3) & ~size_t{3}; }
+// A merge is cut into tasks of 256 elements of an item's group x 128. A device
+// plan holds one arrival counter per (task, item) (block_merge 2), then, on a
+// 16-byte boundary, each item's first unit (block_merge 3): where those start,
+// in int32 elements from the counters.
+constexpr int    merge_tasks(int group) { return group > 2 ? group / 2 : 1; }
+constexpr size_t plan_item_units(int items, int group) {
+    return (static_cast<size_t>(merge_tasks(group)) * static_cast<size_t>(items) + 3) & ~size_t{3};
+}
 
 // Tokens per planning tile (decode.cu:43-45 tile_tokens). The gfx950 kernel
 // consumes 16-token groups, so every 16-token boundary is a legal cut.

@@ -236,7 +236,7 @@ namespace {
 double tile_us(double blocks) { return 0.122 + 0.00071 * blocks; }
 // What merging across blocks adds after a block's last wave, in us: the partial
 // row stored, the arrival, the combine (FP8's blocks hold more rows).
-constexpr double kSpanUs16 = 1.6, kSpanUs32 = 2.4;   // fp16, FP8 (16- and 32-token tiles)
+constexpr double kSpanUs16 = 1.2, kSpanUs32 = 2.0;   // fp16, FP8 (16- and 32-token tiles)
 
 // make_plan's equal cut leaves most items across two or more blocks unless their
 // tiles happen to be whole blocks. Where that costs more than uneven blocks do,
@@ -248,8 +248,8 @@ constexpr double kSpanUs16 = 1.6, kSpanUs32 = 2.4;   // fp16, FP8 (16- and 32-to
 // Same box, us per step, across blocks -> inside: fp16 1 x 200 7.0 -> 5.4, 32 x
 // 200 10.0 -> 7.2, 32 x 1000 24.7 -> 22.3, 32 x 5000 102 -> 97, 128 rows of 100
 // to 200 17.9 -> 16.4; FP8 16 x 200 8.0 -> 5.7, 32 x 2000 25.5 -> 23.0. Left
-// across blocks by the estimate, fp16: 1 x 500 6.9 (8.0 inside), 16 x 500 10.1
-// (11.1), 32 rows of 300 to 1000 17.1 (19.0). Only for the plan that make_plan
+// across blocks by the estimate, fp16: 1 x 500 6.9 (8.0 inside), 16 x 500 9.8
+// (11.1), 32 rows of 300 to 1000 16.6 (19.0). Only for the plan that make_plan
 // gives a grid of its own choice (`units`), whoever brings it: another grid is
 // the caller's. The host plan stays as it is. False: not cut.
 bool cut_in_blocks(const pa_plan& plan, int units, pa_plan& out) {
@@ -447,7 +447,7 @@ void device_plan_upload(pa_device_plan& dp, const pa_plan& plan, int group, int 
     const size_t o_cta   = round4(run.segments.size());
     const size_t o_item  = o_cta + round4(run.cta_seg_begin.size());
     const size_t o_extra = o_item + round4(run.item_seg_begin.size());
-    const size_t o_ctr   = o_extra + round4(n_extra);   // per-item merge counters, uploaded as zeros
+    const size_t o_ctr   = o_extra + round4(n_extra);   // merge counters, uploaded as zeros
     const pa_split_shape& shape = run.shape;
     const int  in_kernel = merge_mode_of(shape, kChainMaxBlocks);
     // Past kChainMaxBlocks: block partials for the merge kernel (block_merge 3),
@@ -457,7 +457,7 @@ void device_plan_upload(pa_device_plan& dp, const pa_plan& plan, int group, int 
     // 9.4; 3 ragged rows to 30000 21.9 / 20.5; 1 x 131072 FP8 46.4 / 45.9.
     const bool blocks    = in_kernel == 0 && merge_mode_of(shape, INT_MAX) == 2 &&
                         (group > 1 || shape.max_blocks >= kOneHeadMinBlocks);
-    const size_t o_unit  = o_ctr + pa::plan_item_units(plan.items);
+    const size_t o_unit  = o_ctr + pa::plan_item_units(plan.items, group);
     const size_t total   = blocks ? o_unit + round4(shape.item_unit.size()) : o_unit;
     if (total > dp.ints_cap) {
         // Growing frees the old block, which decodes queued before may still

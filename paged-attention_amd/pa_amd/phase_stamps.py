@@ -25,10 +25,10 @@ One JSON line per shape:
                      merge's start), lds (the slots' items read), count (wave
                      0's first task found), average (wave 0's tasks: partials
                      read, weighted average computed, its stores issued)
-  store_wait         those partial rows complete at the coherence point
+  store_wait         wave 0's partial rows complete at the coherence point
   arrive             the arrival counter's round trip
-  combine            the last block's combine of an item's block partials:
-                     loads returned / running maximum / lane tree / output
+  combine            where wave 0 is an item's last to arrive: block partials
+                     loaded / averaged / - / output written
   last_end           the last stamp of the step
 
 The phases after `wave_end` exist when the plan merges across blocks inside
