@@ -1278,20 +1278,35 @@ __global__ __launch_bounds__(64 * WAVES) void decode_merge_kernel(const int32_t*
     const int sl = lane / LPS;       // which segment of the wave's pass
     float4 acc = {0.f, 0.f, 0.f, 0.f};
     float  den = 0.f, m = -INFINITY;
-#pragma unroll 4
-    for (int i = wave * SPW + sl; i < n; i += WAVES * SPW) {
-        const size_t sg  = static_cast<size_t>(s0 + (unit0 ? max(0, kWaves * (j0 + i) - u0) : i));
-        const float  lse = part_lse[sg * G + g];
-        const float4 o   = *reinterpret_cast<const float4*>(part_out + (sg * G + g) * kHeadDim + d0 + 4 * dq);
-        const float  mn  = fmaxf(m, lse);
-        const float  f   = exp2_fast(m - mn);      // 0 while m = -inf
-        const float  wgt = exp2_fast(lse - mn);
-        acc.x = fmaf(wgt, o.x, acc.x * f);
-        acc.y = fmaf(wgt, o.y, acc.y * f);
-        acc.z = fmaf(wgt, o.z, acc.z * f);
-        acc.w = fmaf(wgt, o.w, acc.w * f);
-        den   = fmaf(den, f, wgt);
-        m     = mn;
+    // Four segments per lane and round, every load issued before the first is
+    // used. (A loop unrolled by four waits for each load in turn where a lane
+    // has fewer segments, as with block partials: us per step, fp16 1 x 4096
+    // 8.96 -> 8.6, 1 x 16384 15.8 -> 15.5, FP8 1 x 131072 46.2 -> 45.9.)
+    for (int i0 = wave * SPW + sl; i0 < n; i0 += 4 * WAVES * SPW) {
+        float  lse[4];
+        float4 o[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int i = i0 + k * WAVES * SPW;
+            if (i < n) {
+                const size_t sg = static_cast<size_t>(s0 + (unit0 ? max(0, kWaves * (j0 + i) - u0) : i));
+                lse[k] = part_lse[sg * G + g];
+                o[k]   = *reinterpret_cast<const float4*>(part_out + (sg * G + g) * kHeadDim + d0 + 4 * dq);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (i0 + k * WAVES * SPW >= n) break;
+            const float mn  = fmaxf(m, lse[k]);
+            const float f   = exp2_fast(m - mn);      // 0 while m = -inf
+            const float wgt = exp2_fast(lse[k] - mn);
+            acc.x = fmaf(wgt, o[k].x, acc.x * f);
+            acc.y = fmaf(wgt, o[k].y, acc.y * f);
+            acc.z = fmaf(wgt, o[k].z, acc.z * f);
+            acc.w = fmaf(wgt, o[k].w, acc.w * f);
+            den   = fmaf(den, f, wgt);
+            m     = mn;
+        }
     }
     // Combine (m, den, acc) states: lanes of the same dims, then waves. The
     // partner state comes without an LDS round trip: within a row of 16
