@@ -189,6 +189,7 @@ void decode_impl(int dtype, const pa_decode_params& p, hipStream_t s, bool split
 // (which may load the library's code object onto the device) happens at set-up,
 // outside any graph capture of the decode that follows.
 void scratch_prepare();
+size_t scratch_bytes();   // the array's size
 
 // ---- page pool (pa_pool.cpp)
 // Entry i of a batched append: the slot's length before it, and the table

@@ -437,7 +437,13 @@ void device_plan_upload(pa_device_plan& dp, const pa_plan& plan, int group, int 
             throw std::invalid_argument("upload: segment starts must be multiples of 16 tokens");
     const bool kernel_tile = plan.tile == pa::kernel_tile_tokens(PA_KV_FP16, group) ||
                              plan.tile == pa::kernel_tile_tokens(PA_KV_FP8_E4M3, group);
-    const bool snap = kernel_tile && plan.per > 0 && plan_merge_mode(plan) == 2 &&
+    // Cut again only where pa_decode_static's array holds the host plan's
+    // partials: a plan merged in LDS needs none of it, and what that call
+    // refuses does not depend on this cut.
+    const size_t rows  = nseg * static_cast<size_t>(group);
+    const size_t need  = rows * (static_cast<size_t>(head_dim) + 1);
+    const bool   fits  = need * sizeof(float) <= scratch_bytes();
+    const bool   snap  = fits && kernel_tile && plan.per > 0 && plan_merge_mode(plan) == 2 &&
                       cut_in_blocks(plan, device_cus() * pa::kernel_units_per_cu(PA_KV_FP16, group), dp.blocks);
     const pa_plan& run = snap ? dp.blocks : plan;   // what the device gets
     // One block: segments | cta_seg_begin | item_seg_begin | extra | merge
@@ -484,8 +490,6 @@ void device_plan_upload(pa_device_plan& dp, const pa_plan& plan, int group, int 
     dp.item_seg_begin = dp.ints + o_item;
     dp.extra          = n_extra ? dp.ints + o_extra : nullptr;
     dp.merge_counters = dp.ints + o_ctr;
-    const size_t rows = nseg * static_cast<size_t>(group);
-    const size_t need = rows * (static_cast<size_t>(head_dim) + 1);
     if (need > dp.part_cap) {
         pa::hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");   // queued decodes may still use it
         pa::hip_check(hipFree(dp.partial_out), "hipFree");

@@ -65,6 +65,7 @@ using namespace pa::host;
 
 namespace pa::host {
 void scratch_prepare() { (void)scratch_on_current_device(true); }
+size_t scratch_bytes() { return kScratchBytes; }
 }  // namespace pa::host
 
 extern "C" {

@@ -85,6 +85,27 @@ def _device_plan_arrays(p, items):
     return cta, item, d2h(int(p.segments), 16 * int(cta[-1]), np.int32).reshape(-1, 4)
 
 
+def test_decode_static_refuses_the_same_plans():
+    """A plan whose partials exceed the static workspace keeps its rows across blocks, and is refused there."""
+    import torch
+    lens = [17 + (i * 37) % 48 for i in range(1024)]
+    q, k, v, table, ks, vs = paged_inputs(len(lens), lens, 64, 8, 16, False, seed=5)
+    plan = _plan(False, lens, 8, 8, 0)
+    assert plan.merge_mode == 2 and len(plan.segments) * 8 * (D + 1) * 4 > 32 << 20
+    dplan = pa_amd.DevicePlan()
+    dplan.upload(plan, 8, D)
+    p = pa_amd.DecodeParams()
+    dplan.bind(p)
+    out = torch.empty_like(q)
+    p.q, p.k_cache, p.v_cache, p.block_table = q.data_ptr(), k.data_ptr(), v.data_ptr(), table.data_ptr()
+    p.out, p.block_table_stride = out.data_ptr(), table.size(1)
+    p.batch, p.num_q_heads, p.num_kv_heads, p.head_dim, p.page_size = len(lens), 64, 8, D, 16
+    p.sm_scale, p.k_scale, p.v_scale = pa_amd.sm_scale(D), ks, vs
+    assert p.block_merge == 2
+    lib = pa_amd._lib.load()
+    assert lib.pa_decode_static(pa_amd.FP16, ctypes.byref(p), p.num_segments, None) == pa_amd._lib.PA_ERR_LENGTH
+
+
 @pytest.mark.parametrize("lens,fp8,group,hkv", [
     ([200], False, 4, 8),                          # one item per block, fewer blocks than the chip has
     ([33], False, 2, 8),                           # three tiles per item
