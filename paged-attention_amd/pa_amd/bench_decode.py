@@ -268,7 +268,7 @@ def append_rows(batch: int, hkv: int, dim: int, page: int, fp8: bool, steps: int
     """Cost of growing the cache (paged_kv_cache.cu:95-136). A decode step
     appends one token to each of `batch` sequences: `batch` append calls (each
     synchronizes its stream, as the reference's) against one append_batch call
-    (one pinned copy + one kernel, no synchronization); wall time per step over
+    (one kernel, no synchronization); wall time per step over
     `steps` steps. Then a prefill of `prefill` tokens per sequence through one
     append_batch call, timed with events (host staging and its copy included;
     median of 5); bytes = fp16 K and V read + K and V written at the cache's

@@ -343,8 +343,9 @@ class PagedKVCache:
         return bool(done.value)
 
     def append_batch(self, slots, counts, k, v, stream=None) -> bool:
-        """Appends counts[i] tokens to slots[i] for every i in one copy + one
-        kernel; k / v hold the tokens concatenated in entry order
+        """Appends counts[i] tokens to slots[i] for every i in one kernel
+        (its metadata in the arguments; past 896 ints a copy kernel brings it);
+        k / v hold the tokens concatenated in entry order
         ([sum(counts)][Hkv][D] fp16, device). All-or-nothing on pages."""
         slots = np.ascontiguousarray(slots, dtype=np.int32)
         counts = np.ascontiguousarray(counts, dtype=np.int32)
