@@ -392,6 +392,7 @@ EXTRA = [("c1", "c1", 16, True), ("c3", "c3", 16, True), ("c2_p16", "c2", 16, Tr
 
 
 MERGE_NAMES = {0: "merge kernel", 1: "in the split kernel, inside one block",
+               4: "in the split kernel, inside one block",
                2: "in the split kernel, across blocks",
                3: "per block in the split kernel, then the merge kernel"}
 

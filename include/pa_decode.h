@@ -78,7 +78,7 @@ typedef struct pa_decode_params {
     int32_t         max_item_segments; /* most segments of one (row, kv head); sizes the
                                           merge launch (0 = unknown). Set by bind. */
     int32_t         block_merge;       /* How the split kernel merges split (row, kv head)
-                                          items itself (needs_merge is then 0 for 1 and 2,
+                                          items itself (needs_merge is then 0 for 1, 2 and 4,
                                           which the launches refuse together with it, and 1
                                           for 3). Set by bind.
                                           0: it does not (the merge kernel does, if
@@ -90,7 +90,9 @@ typedef struct pa_decode_params {
                                           finish (merge_counters) combines them.
                                           3: each block writes such partials as under 2 and
                                           the merge kernel combines them (items over more
-                                          blocks than 2 takes). */
+                                          blocks than 2 takes).
+                                          4: as 1, every tile of a segment scored against its
+                                          own maximum (segments joined from single tiles). */
     int32_t         num_segments;      /* segments of the bound plan (0 = unknown); sizes the
                                           partial workspace. Set by bind. */
     int32_t*        merge_counters;    /* block_merge 2: arrival counters (one per item and 256
@@ -194,7 +196,7 @@ pa_status pa_decode_merge(int dtype, const pa_decode_params* p, void* stream);
  * PA_ERR_INVALID_ARGUMENT before any launch. A plan whose workspace,
  * num_segments * group * (head_dim + 1) * 4 bytes, exceeds 32 MiB is refused
  * with PA_ERR_LENGTH; plans without split rows, or merged in the split kernel
- * (p->block_merge = 1), need none. The array's address is looked up by the
+ * (p->block_merge = 1 or 4), need none. The array's address is looked up by the
  * plan upload on the device (so a first call made under graph capture needs
  * no lookup); a first call on a device that has seen no upload looks it up
  * itself, and refuses to while its stream is being captured. Allocates

@@ -54,7 +54,7 @@
 //     through a per-wave LDS slot once per segment; on the LDS-stage paths it
 //     lands there with the same LDS-destination loads, ahead of the K / V.
 //   * Split rows are merged by the split kernel itself when the plan allows
-//     (block_merge 1 and 2): a unit's split segments are only its first and
+//     (block_merge 1, 2 and 4): a unit's split segments are only its first and
 //     last, so each wave keeps at most two partials (and their LSEs) in LDS;
 //     after one barrier the waves merge the block's split rows side by side
 //     (tasks of 256 elements of one row). A row inside the block (e.g. 32 rows x 8 kv heads x
@@ -174,6 +174,10 @@ namespace {
 
 constexpr int   kWaves        = kBlockUnits;   // waves (work units) per block
 constexpr float kRescaleSlack = 8.0f;   // log2 headroom of the lazy running max
+// How far below the running maximum a tile's own one is followed (block_merge
+// 4; log2): what a tile further below adds is lost in 32 bits anyway, and the
+// sums grow by at most 2^32 at each of the few tiles of such a segment.
+constexpr float kTileMaxDrop = 32.0f;
 constexpr float kLog2e        = 1.4426950408889634f;
 // The cache-policy operand of buffer loads (2 = non-temporal).
 template <bool NT> constexpr int kAux = NT ? 2 : 0;
@@ -359,7 +363,7 @@ struct alignas(16) Slot {
 // 32 x 1024) is level. Eight elements per lane (half the tasks) were 0.3 us
 // slower where a block holds one or two runs and no faster elsewhere.
 //
-// An item whose segments all lie in this block (block_merge 1: every split
+// An item whose segments all lie in this block (block_merge 1 and 4: every split
 // item) is written as fp16. With block_merge 2 and 3 an item may also span blocks
 // (its k-th segment runs in unit u0 + k, so it continues from the previous
 // block at the block's first slot and into the next at its last): the block's
@@ -386,7 +390,7 @@ __device__ __forceinline__ void block_merge(const pa_decode_params& p, const Slo
     static_assert(NS == 16, "the slots fit the low lanes of a wave");
     const int  lane  = tid & 63;
     const int  wave  = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const bool chain = p.block_merge >= 2;
+    const bool chain = p.block_merge == 2 || p.block_merge == 3;
     if (tid == 0) stamp(16);
     const Slot     mine   = slots[lane & (NS - 1)];   // lane j holds slot j
     const uint32_t filled = static_cast<uint32_t>(__builtin_amdgcn_ballot_w64(lane < NS && mine.item >= 0));
@@ -596,6 +600,13 @@ __device__ __forceinline__ void decode_split_body(const pa_decode_params& p, con
     const int lblock = static_cast<int>(blockIdx.x);   // units 8 lblock .. 8 lblock + 7
     const int unit   = lblock * kWaves + wave;
     const bool merge_here = p.block_merge != 0;   // block-level merge of split rows
+    // block_merge 4: every step is scored against its own maximum, as if it were
+    // a segment of its own. (Segments of one tile each are that, but a segment
+    // costs a chain of its own, its Q, its counts, its partial: one row of 200, 13
+    // tiles over 8 waves, 6.9 us as segments, 5.6 as this, 6.4 across blocks.)
+    const bool  tile_max = p.block_merge == 4;
+    const float slack    = tile_max ? -INFINITY : kRescaleSlack;
+    const float drop     = tile_max ? kTileMaxDrop : 0.f;
     if (lane == 0) {
         slots[2 * wave].item     = -1;
         slots[2 * wave + 1].item = -1;
@@ -936,7 +947,7 @@ __device__ __forceinline__ void decode_split_body(const pa_decode_params& p, con
     auto rescale = [&](float xmax) {
         float mx = fmaxf(xmax, __shfl_xor(xmax, 16));
         mx = fmaxf(mx, __shfl_xor(mx, 32));
-        const float m_new = fmaxf(m_run, mx);
+        const float m_new = fmaxf(m_run - drop, mx);
         const float alpha = exp2_fast(m_run - m_new);
         m_run = m_new;
         l_run *= alpha;
@@ -1050,7 +1061,7 @@ __device__ __forceinline__ void decode_split_body(const pa_decode_params& p, con
         }
         float xmax = fmaxf(fmaxf(x[0][0], x[0][1]), fmaxf(x[0][2], x[0][3]));
         if constexpr (NH > 1) xmax = fmaxf(xmax, fmaxf(fmaxf(x[1][0], x[1][1]), fmaxf(x[1][2], x[1][3])));
-        if (__builtin_expect(__builtin_amdgcn_ballot_w64(c < G && xmax > m_run + kRescaleSlack) != 0, 0))
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(c < G && xmax > m_run + slack) != 0, 0))
             rescale(xmax);
         float pr[NH][4];
         float psum = 0.f;
@@ -1540,7 +1551,7 @@ int kernel_units_per_cu(int dtype, int group) {
 }
 
 // A plan's split rows are merged either by the merge kernel (needs_merge) or
-// inside the split kernel (block_merge 1 and 2), never both: the workspace then
+// inside the split kernel (block_merge 1, 2 and 4), never both: the workspace then
 // holds partial rows only at the slots the split kernel merges through, and the
 // merge kernel would read the others unwritten. (Under block_merge 3 it reads
 // those slots only.)
@@ -1561,8 +1572,8 @@ hipError_t launch_decode_split(int dtype, const pa_decode_params& p, hipStream_t
         throw std::invalid_argument("decode: null pointer in params");
     if ((p.needs_merge || p.block_merge) && (!p.partial_out || !p.partial_lse))
         throw std::invalid_argument("decode: split rows need the partial workspace");
-    if (p.block_merge < 0 || p.block_merge > 3) throw std::invalid_argument("decode: block_merge must be 0, 1, 2 or 3");
-    if (p.block_merge >= 2 && !p.merge_counters)
+    if (p.block_merge < 0 || p.block_merge > 4) throw std::invalid_argument("decode: block_merge must be 0 to 4");
+    if ((p.block_merge == 2 || p.block_merge == 3) && !p.merge_counters)
         throw std::invalid_argument("decode: block_merge 2 and 3 need the plan's merge counters");
     return dtype == PA_KV_FP16 ? launch_split_e<2>(p, g, s) : launch_split_e<1>(p, g, s);
 }

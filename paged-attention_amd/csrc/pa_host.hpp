@@ -82,7 +82,7 @@ struct pa_device_plan {
     int      num_segments = 0;
     int      block_merge = 0;          // pa_decode_params.block_merge of the plan
     int32_t* merge_counters = nullptr;  // arrival counters in `ints`
-    pa_plan  blocks;                    // the plan cut again inside blocks, where that is what runs
+    pa_plan  blocks;                    // the plan grouped inside blocks, where that is what runs
     pa_stage_pool staging;
 };
 

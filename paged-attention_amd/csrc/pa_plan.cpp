@@ -234,107 +234,135 @@ namespace {
 // the two the measured time is linear (rows of 500 tokens, fp16, one block per
 // (row, kv head): 8 blocks 67 GB/s per CU, 32 52, 128 36).
 double tile_us(double blocks) { return 0.122 + 0.00071 * blocks; }
+// Tiles of one item joined in a segment at most (block_merge 4).
+constexpr int kMaxJoined = 3;
 // What merging across blocks adds after a block's last wave, in us: the partial
 // row stored, the arrival, the combine (FP8's blocks hold more rows).
 constexpr double kSpanUs16 = 1.2, kSpanUs32 = 2.0;   // fp16, FP8 (16- and 32-token tiles)
 
 // make_plan's equal cut leaves most items across two or more blocks unless their
-// tiles happen to be whole blocks. Where that costs more than uneven blocks do,
-// the plan runs cut again so that no item spans blocks: every block takes whole
-// items (one each where there are no more items than blocks, else runs of them
-// with the smallest largest block), in equal ranges over its units. The
-// estimates of both: the plan's blocks are equal; uneven ones run together for
-// the average block and the rest of the largest at less than half of them.
-// Same box, us per step, across blocks -> inside: fp16 1 x 200 7.0 -> 5.4, 32 x
-// 200 10.0 -> 7.2, 32 x 1000 24.7 -> 22.3, 32 x 5000 102 -> 97, 128 rows of 100
-// to 200 17.9 -> 16.4; FP8 16 x 200 8.0 -> 5.7, 32 x 2000 25.5 -> 23.0. Left
-// across blocks by the estimate, fp16: 1 x 500 6.9 (8.0 inside), 16 x 500 9.8
-// (11.1), 32 rows of 300 to 1000 16.6 (19.0). Only for the plan that make_plan
-// gives a grid of its own choice (`units`), whoever brings it: another grid is
-// the caller's. The host plan stays as it is. False: not cut.
-bool cut_in_blocks(const pa_plan& plan, int units, pa_plan& out) {
+// tiles happen to be whole blocks. Where that costs more than uneven units do,
+// its segments run on other units, so that no item spans blocks: whole items per
+// block (one each where there are no more items than blocks), a unit's segments
+// consecutive, at most `limit` tiles of them (the smallest that fits) and only the
+// first and last of them split ones (the kernel's two LDS slots).
+// A segment's probabilities are rounded to 16 bits against its own running
+// maximum, so the segments stay the plan's own, in units of their own: longer
+// ones would lose precision. Where the plan's are single tiles, a unit's tiles of
+// one item are joined, and the kernel takes each against its own maximum
+// (block_merge 4): the same probabilities, bit for bit. (Joined without that, one
+// row of 200 lay 2.65e-4 from 64 bits instead of 2.46e-4.)
+// The estimates of both: the plan's blocks are equal; uneven ones run together for
+// the average block and the rest of the largest at less than half of them. Same
+// box, us per decode, 50 in a graph, across blocks -> inside: joined tiles, fp16
+// 1 x 33 6.0 -> 4.1, 1 x 200 6.4 -> 5.6, 16 x 200 7.6 -> 6.2, FP8 16 x 200 7.6 ->
+// 5.9, 1 x 400 7.1 -> 6.7; the plan's segments, fp16 32 x 200 9.2 -> 6.6, 64 x 200
+// 12.9 -> 10.1, FP8 120 rows of 95 to 161 10.1 -> 8.1, 32 x 1100 14.7 -> 14.5. Left
+// across blocks by the estimate, for longer segments inside would cost precision
+// and uneven units time: fp16 32 x 1000, 32 x 5000, 128 rows of 100 to 200, FP8 32 x
+// 2000 (22.3, 97, 16.4 and 23.0 when segments were cut anew; 24.7, 102, 17.9, 25.5).
+// Only for the plan that make_plan gives a grid of its own choice (`units`), whoever
+// brings it: another grid is the caller's. The host plan stays as it is.
+// False: not grouped, `out` holds nothing of use.
+bool group_in_blocks(const pa_plan& plan, int units, pa_plan& out) {
     const int items = plan.items, max_blocks = units / pa::kBlockUnits;
     if (items <= 0 || max_blocks <= 0 || plan.per <= 0) return false;
-    std::vector<int32_t> tiles(static_cast<size_t>(items));
-    int  longest = 0;
-    long total   = 0;
+    auto tiles = [&](int sg) {
+        const int32_t* s = &plan.segments[4 * static_cast<size_t>(sg)];
+        return (s[3] - s[2] + plan.tile - 1) / plan.tile;
+    };
+    long longest = 0, total = 0;
     for (int i = 0; i < items; ++i) {
-        const int len = plan.segments[4 * static_cast<size_t>(plan.item_seg_begin[i + 1]) - 1];
-        tiles[static_cast<size_t>(i)] = (len + plan.tile - 1) / plan.tile;
-        longest = std::max(longest, tiles[static_cast<size_t>(i)]);
-        total += tiles[static_cast<size_t>(i)];
+        const int  len = plan.segments[4 * static_cast<size_t>(plan.item_seg_begin[i + 1]) - 1];
+        const long t   = (len + plan.tile - 1) / plan.tile;
+        longest = std::max(longest, t);
+        total += t;
     }
     if (plan.per != (total + units - 1) / units) return false;
     const double across = static_cast<double>(pa::kBlockUnits) * plan.per * tile_us(plan.num_ctas / 8.0) +
                           (plan.tile == 16 ? kSpanUs16 : kSpanUs32);
-    auto inside = [&](long largest, int blocks) {
-        const double mean = static_cast<double>(total) / blocks;
-        return mean * tile_us(blocks) + (static_cast<double>(largest) - mean) * tile_us(0.4 * blocks);
+    auto inside = [&](int limit, int blocks) {
+        const double mean    = static_cast<double>(total) / blocks;
+        const double largest = static_cast<double>(std::max<long>(longest, static_cast<long>(pa::kBlockUnits) * limit));
+        return mean * tile_us(blocks) + (largest - mean) * tile_us(0.4 * blocks);
     };
     const bool one_each = items <= max_blocks;
-    long cap = longest;
-    if (one_each) {
-        if (inside(longest, items) >= across) return false;
-    } else {
-        // The smallest cap, to 1/32, under which greedy runs need no more blocks.
-        cap = std::max<long>(cap, (total + max_blocks - 1) / max_blocks);
-        for (;; cap += cap / 32 + 1) {
-            if (inside(cap, max_blocks) >= across) return false;
-            int  blocks = 0;
-            long left   = 0;
-            for (const int32_t t : tiles) {
-                if (t > left) ++blocks, left = cap;
-                left -= t;
+    const bool join     = plan.per == 1;
+    // Units as prefixes of the plan's segments: the last entry is the open one,
+    // with `load` tiles in `count` segments, the last of a split item or not.
+    auto& cta = out.cta_seg_begin;
+    int  limit = plan.per, load = 0, count = 0;
+    bool last_split = false;
+    auto block_begins = [&] { return count == 0 && (cta.size() - 1) % pa::kBlockUnits == 0; };
+    auto close_block = [&](int sg) {
+        do cta.push_back(sg);
+        while ((cta.size() - 1) % pa::kBlockUnits != 0);
+        load = count = 0;
+    };
+    auto place = [&](int i) {   // false: the block has no unit left for item i
+        const int first = plan.item_seg_begin[i], end = plan.item_seg_begin[i + 1];
+        for (int sg = first; sg < end; ++sg) {
+            const int  t    = tiles(sg);
+            const bool more = sg > first && count > 0;   // the unit's last segment is the item's too
+            if (count > 0 && (load + t > limit || (more ? !join : count > 1 && last_split))) {
+                if (cta.size() % pa::kBlockUnits == 0) return false;
+                cta.push_back(sg);
+                load = count = 0;
+            } else if (more) {
+                --count;   // joined
             }
-            if (blocks <= max_blocks) break;
+            load += t;
+            ++count;
+            last_split = end - first > 1;
         }
+        return true;
+    };
+    auto fill = [&] {
+        cta.assign(1, 0);
+        load = count = 0;
+        for (int i = 0; i < items; ++i) {
+            const size_t at = cta.size();
+            const bool begins = block_begins();
+            if (!begins && one_each) close_block(plan.item_seg_begin[i]);
+            else if (place(i)) continue;
+            else if (begins) return false;
+            else {
+                cta.resize(at);
+                close_block(plan.item_seg_begin[i]);
+            }
+            if (cta.size() > static_cast<size_t>(units) || !place(i)) return false;
+        }
+        return true;
+    };
+    for (;; limit += limit / 8 + 1) {
+        if ((join && limit > kMaxJoined) || inside(limit, one_each ? items : max_blocks) >= across) return false;
+        if (fill()) break;
     }
-    out.num_ctas = 0;
-    out.tile     = plan.tile;
-    out.items    = items;
-    out.shape    = {};
+    close_block(plan.item_seg_begin[items]);   // its last entry ends the last unit
+    out.num_ctas = static_cast<int>(cta.size()) - 1;
+    if (inside(limit, out.num_ctas / pa::kBlockUnits) >= across) return false;
+    out.shape = {};
     out.segments.clear();
-    out.cta_seg_begin.clear();
     out.segments.reserve(plan.segments.size());
-    out.item_seg_begin.resize(static_cast<size_t>(items) + 1);
-    for (int i = 0; i < items;) {
-        int  end  = i + 1;
-        long load = tiles[static_cast<size_t>(i)];
-        while (!one_each && end < items && load + tiles[static_cast<size_t>(end)] <= cap)
-            load += tiles[static_cast<size_t>(end++)];
-        const long per = (load + pa::kBlockUnits - 1) / pa::kBlockUnits;
-        long left = per;
-        out.cta_seg_begin.push_back(static_cast<int32_t>(out.segments.size() / 4));
-        for (; i < end; ++i) {
-            const size_t  last  = 4 * static_cast<size_t>(plan.item_seg_begin[i + 1]) - 4;   // the item's last segment
-            const int     row = plan.segments[last], head = plan.segments[last + 1], len = plan.segments[last + 3];
-            const int32_t first = static_cast<int32_t>(out.segments.size() / 4);
-            out.item_seg_begin[static_cast<size_t>(i)] = first;
-            for (long done = 0; done < tiles[static_cast<size_t>(i)];) {
-                if (left == 0) {
-                    out.cta_seg_begin.push_back(static_cast<int32_t>(out.segments.size() / 4));
-                    left = per;
-                }
-                const long take = std::min<long>(left, tiles[static_cast<size_t>(i)] - done);
-                out.segments.insert(out.segments.end(),
-                                    {row, head, static_cast<int32_t>(done * plan.tile),
-                                     static_cast<int32_t>(std::min<long>((done + take) * plan.tile, len))});
-                done += take;
-                left -= take;
+    out.item_seg_begin.assign(static_cast<size_t>(items) + 1, 0);
+    for (int u = 0, item = 0, sg = 0, begin = 0; u < out.num_ctas; ++u) {
+        const int end = cta[static_cast<size_t>(u) + 1];
+        for (cta[static_cast<size_t>(u)] = begin; sg < end; ++sg) {
+            const bool first = sg == plan.item_seg_begin[item + 1];
+            if (first) out.item_seg_begin[static_cast<size_t>(++item)] = begin;
+            const int32_t* s = &plan.segments[4 * static_cast<size_t>(sg)];
+            if (!first && join && begin > cta[static_cast<size_t>(u)]) {
+                out.segments.back() = s[3];
+            } else {
+                out.segments.insert(out.segments.end(), s, s + 4);
+                ++begin;
             }
-            const int n = static_cast<int>(out.segments.size() / 4) - first;
+            const int n = begin - out.item_seg_begin[static_cast<size_t>(item)];
             out.shape.max_segments = std::max(out.shape.max_segments, n);
-            if (n > 1) out.shape.split = true, out.shape.max_blocks = 1;
         }
-        // The block's unused units are empty.
-        out.num_ctas += pa::kBlockUnits;
-        out.cta_seg_begin.resize(static_cast<size_t>(out.num_ctas), static_cast<int32_t>(out.segments.size() / 4));
     }
-    const int32_t nseg = static_cast<int32_t>(out.segments.size() / 4);
-    out.item_seg_begin[static_cast<size_t>(items)] = nseg;
-    out.cta_seg_begin.push_back(nseg);
-    // The workspace (used if a caller forces the merge kernel) holds the plan's count.
-    return out.segments.size() <= plan.segments.size();
+    cta.back() = out.item_seg_begin.back() = static_cast<int32_t>(out.segments.size() / 4);
+    return true;
 }
 }  // namespace
 namespace {
@@ -437,15 +465,15 @@ void device_plan_upload(pa_device_plan& dp, const pa_plan& plan, int group, int 
             throw std::invalid_argument("upload: segment starts must be multiples of 16 tokens");
     const bool kernel_tile = plan.tile == pa::kernel_tile_tokens(PA_KV_FP16, group) ||
                              plan.tile == pa::kernel_tile_tokens(PA_KV_FP8_E4M3, group);
-    // Cut again only where pa_decode_static's array holds the host plan's
-    // partials: a plan merged in LDS needs none of it, and what that call
-    // refuses does not depend on this cut.
+    // Grouped only where pa_decode_static's array holds the plan's partials: a
+    // plan merged in LDS needs none of it, and what that call refuses does not
+    // depend on the grouping.
     const size_t rows  = nseg * static_cast<size_t>(group);
     const size_t need  = rows * (static_cast<size_t>(head_dim) + 1);
     const bool   fits  = need * sizeof(float) <= scratch_bytes();
-    const bool   snap  = fits && kernel_tile && plan.per > 0 && plan_merge_mode(plan) == 2 &&
-                      cut_in_blocks(plan, device_cus() * pa::kernel_units_per_cu(PA_KV_FP16, group), dp.blocks);
-    const pa_plan& run = snap ? dp.blocks : plan;   // what the device gets
+    const bool   inside = fits && kernel_tile && plan.per > 0 && plan_merge_mode(plan) == 2 &&
+                        group_in_blocks(plan, device_cus() * pa::kernel_units_per_cu(PA_KV_FP16, group), dp.blocks);
+    const pa_plan& run = inside ? dp.blocks : plan;   // what the device gets
     // One block: segments | cta_seg_begin | item_seg_begin | extra | merge
     // counters, each part starting on a 16-byte boundary (the kernels read
     // segments as int4).
@@ -455,7 +483,7 @@ void device_plan_upload(pa_device_plan& dp, const pa_plan& plan, int group, int 
     const size_t o_extra = o_item + round4(run.item_seg_begin.size());
     const size_t o_ctr   = o_extra + round4(n_extra);   // merge counters, uploaded as zeros
     const pa_split_shape& shape = run.shape;
-    const int  in_kernel = merge_mode_of(shape, kChainMaxBlocks);
+    const int  in_kernel = !inside ? merge_mode_of(shape, kChainMaxBlocks) : plan.per == 1 ? 4 : 1;
     // Past kChainMaxBlocks: block partials for the merge kernel (block_merge 3),
     // where the split kernel can find an item's part of a block. Same box, us per
     // step, every segment's partial / block partials: one row of 131072, one kv

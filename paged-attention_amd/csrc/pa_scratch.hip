@@ -95,7 +95,7 @@ pa_status pa_decode_static(int dtype, const pa_decode_params* p, int num_segment
         // kernel (block_merge 2), write partials to the workspace, at most
         // rows * (head_dim + 1) floats; plans merged inside one block keep
         // theirs in LDS, and plans without split rows write none.
-        const bool   hbm_partials = split_rows && p->block_merge != 1;
+        const bool   hbm_partials = split_rows && p->block_merge != 1 && p->block_merge != 4;
         const size_t need = hbm_partials ? rows * (static_cast<size_t>(pa::kHeadDim) + 1) * sizeof(float) : 0;
         if (need > kScratchBytes)
             throw std::length_error("decode_static: the plan's partial workspace (" + std::to_string(need) +

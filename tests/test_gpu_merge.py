@@ -112,39 +112,93 @@ def test_decode_static_refuses_the_same_plans():
     ([200] * 32, False, 4, 8),                     # as many items as blocks
     ([1100] * 32, True, 8, 8),
     ([10, 33, 300, 1, 64, 250, 17, 129], True, 1, 8),
-    ([100, 150, 200, 130, 170, 110, 190, 120] * 16, False, 4, 8),   # several items per block
+    ([200] * 64, False, 4, 8),                     # two items per block
     ([1, 9, 33, 20, 16, 31, 2, 40, 17] * 6, False, 8, 8),           # many short items per block
     ([95, 161, 128] * 40, True, 4, 4),
 ], ids=["row", "three_tiles", "full", "g8", "ragged", "packed", "short", "fp8_packed"])
 def test_items_kept_inside_blocks(lens, fp8, group, hkv):
-    """Plans of make_plan's own grid whose items would straddle blocks run cut again: every block of 8 units
-    holds whole items, every token once and in order, and the decode matches the oracle and the merge kernel."""
+    """Plans of make_plan's own grid whose items would straddle blocks run on other units: every block of 8 units
+    holds whole items, an item's segments lie in consecutive units, a unit's split ones are its first and last, and
+    the decode matches the oracle and the merge kernel. The segments stay the plan's own (block_merge 1), or, where
+    those are single tiles, runs of two or three of them (block_merge 4)."""
     plan = _plan(fp8, lens, group, hkv, 0)
     assert plan.merge_mode == 2
+    tile, host, items = 32 if fp8 else 16, np.asarray(plan.segments), len(lens) * hkv
+    single = bool(np.all(host[:, 3] - host[:, 2] <= tile))
     dplan = pa_amd.DevicePlan()
     dplan.upload(plan, group, D)
     p = pa_amd.DecodeParams()
     dplan.bind(p)
-    assert p.block_merge == 1 and p.num_segments == len(plan.segments) and p.num_ctas % 8 == 0
-    cta, item, seg = _device_plan_arrays(p, len(lens) * hkv)
-    assert len(seg) <= len(plan.segments) and np.all(np.diff(cta) >= 0) and item[-1] == len(seg)
+    assert p.block_merge == (4 if single else 1)
+    assert p.num_segments == len(host) and p.num_ctas % 8 == 0
+    cta, item, seg = _device_plan_arrays(p, items)
+    if single:
+        assert np.all(seg[:, 3] - seg[:, 2] <= 3 * tile)
+    else:
+        assert np.array_equal(seg, host)
+    assert cta[0] == 0 and cta[-1] == len(seg) and np.all(np.diff(cta) >= 0)
     unit = np.repeat(np.arange(p.num_ctas), np.diff(cta))
-    for i in range(len(lens) * hkv):
+    split = np.repeat(np.diff(item) > 1, np.diff(item))
+    for i in range(items):
         rows = seg[item[i]:item[i + 1]]
         assert len(rows) and np.all(rows[:, 0] == i // hkv) and np.all(rows[:, 1] == i % hkv)
         assert rows[0, 2] == 0 and rows[-1, 3] == lens[i // hkv] and np.array_equal(rows[1:, 2], rows[:-1, 3])
+        assert np.all(rows[:, 2] % tile == 0)
         u = unit[item[i]:item[i + 1]]
         assert u[0] // 8 == u[-1] // 8 and np.array_equal(u, np.arange(u[0], u[0] + len(u)))
-    for u in range(p.num_ctas):     # a unit's split segments are its first and last
-        split = [s for s in range(cta[u], cta[u + 1]) if np.sum(unit[item[seg[s, 0] * hkv + seg[s, 1]]:
-                                                                   item[seg[s, 0] * hkv + seg[s, 1] + 1]] >= 0) > 1]
-        assert all(s in (cta[u], cta[u + 1] - 1) for s in split)
-    _check(fp8, lens, group, hkv, plan.handle.value, 1, repeats=2)
+    for u in range(p.num_ctas):
+        assert not split[cta[u] + 1:cta[u + 1] - 1].any()
+    _check(fp8, lens, group, hkv, plan.handle.value, p.block_merge, repeats=2)
+
+
+@pytest.mark.parametrize("lens,fp8,group,hkv", [
+    ([200], False, 4, 8),                          # 13 tiles in 8 units
+    ([199, 250, 33], True, 8, 8),
+    ([200] * 32, False, 4, 8),
+    ([1, 9, 33, 20, 16, 31, 2, 40, 17] * 6, False, 2, 8),
+], ids=["row", "ragged", "full", "short"])
+def test_grouping_keeps_the_partials(lens, fp8, group, hkv):
+    """Inside blocks or across them, the decode averages the same partials. With partials equal bit for bit, two
+    fp32 averages of at most 16 of them (weights in [0, 1], values below 4.5) differ by at most 16 * 2^-24 * 4.5,
+    so two fp16 results differ by one rounding at most, and only where the average lies that near to the middle of
+    two fp16 values: 2 * 4.3e-6 of the spacing 2^-13 of values above 1/8, under 2^-3 of the results at worst."""
+    import torch
+    hq, dt = hkv * group, pa_amd.FP8_E4M3 if fp8 else pa_amd.FP16
+    q, k, v, table, ks, vs = paged_inputs(len(lens), lens, hq, hkv, 16, fp8, seed=11)
+    plan = _plan(fp8, lens, group, hkv, 0)
+    # The same units behind an empty one: no cut that make_plan gives, so it runs as it is.
+    cta = np.concatenate([[0], plan.cta_seg_begin]).astype(np.int32)
+    seg, item = np.ascontiguousarray(plan.segments), np.ascontiguousarray(plan.item_seg_begin)
+    h = ctypes.c_void_p()
+    pa_amd._lib.call("pa_plan_create", len(cta) - 1, plan.tile, seg.ctypes.data, len(seg), cta.ctypes.data,
+                     item.ctypes.data, len(item) - 1, hkv, ctypes.byref(h))
+    outs = []
+    try:
+        for handle, modes in ((plan.handle.value, (1, 4)), (h.value, (2,))):
+            dplan = pa_amd.DevicePlan()
+            pa_amd._lib.call("pa_device_plan_upload", dplan._h, handle, group, D, None)
+            p = pa_amd.DecodeParams()
+            out = torch.empty_like(q)
+            p.q, p.k_cache, p.v_cache, p.block_table = q.data_ptr(), k.data_ptr(), v.data_ptr(), table.data_ptr()
+            p.out, p.block_table_stride = out.data_ptr(), table.size(1)
+            p.batch, p.num_q_heads, p.num_kv_heads, p.head_dim, p.page_size = len(lens), hq, hkv, D, 16
+            p.sm_scale, p.k_scale, p.v_scale = pa_amd.sm_scale(D), ks, vs
+            dplan.bind(p)
+            assert p.block_merge in modes
+            pa_amd.paged_decode(dt, p)
+            torch.cuda.synchronize()
+            outs.append(out.float())
+    finally:
+        pa_amd._lib.load().pa_plan_destroy(h.value)
+    apart = (outs[0] - outs[1]).abs()
+    assert float(apart.max()) <= 2.0 ** -9
+    assert float((apart > 0).float().mean()) < 2.0 ** -3
 
 
 def test_another_grid_is_left_as_it_is():
     """A caller's grid, and rows that are cheaper across blocks, keep the host plan's arrays."""
-    for lens, ctas in (([200] * 32, 512), ([500], 0), ([300, 1000, 450, 700] * 8, 0)):
+    for lens, ctas in (([200] * 32, 512), ([500], 0), ([300, 1000, 450, 700] * 8, 0),
+                       ([100, 150, 200, 130, 170, 110, 190, 120] * 16, 0)):
         plan = _plan(False, lens, 4, 8, ctas)
         assert plan.merge_mode == 2
         dplan = pa_amd.DevicePlan()
