@@ -85,6 +85,9 @@ pa_status pa_decode_static(int dtype, const pa_decode_params* p, int num_segment
         if (num_segments != p->num_segments)
             throw std::invalid_argument("decode_static: num_segments (" + std::to_string(num_segments) +
                                         ") differs from the bound plan's (" + std::to_string(p->num_segments) + ")");
+        // The count is the host plan's, also where the device plan has its
+        // segments grouped inside blocks: that one says so by block_merge 1 or 4,
+        // whether it left an item in several segments or not.
         const long items      = static_cast<long>(p->batch) * p->num_kv_heads;
         const bool split_rows = p->num_segments > items;
         if (split_rows && (!p->block_merge || p->block_merge == 3) && !p->needs_merge)

@@ -107,6 +107,48 @@ def test_decode_static_refuses_the_same_plans():
 
 
 @pytest.mark.parametrize("lens,fp8,group,hkv", [
+    ([48] * 165, False, 4, 8),
+    ([192] * 203, True, 4, 8),
+    ([1344] * 248, True, 4, 8),
+    ([112] * 385, False, 4, 4),
+    ([200] * 32, False, 4, 8),
+    ([200], False, 8, 8),
+    ([33, 17, 48], True, 1, 8),
+], ids=["165x48", "203x192_fp8", "248x1344_fp8", "385x112", "32x200", "row", "ragged"])
+def test_decode_static_takes_grouped_plans(lens, fp8, group, hkv):
+    """Plans whose host copy has split rows, grouped inside blocks or not: the allocation-free entry point takes
+    them and gives what the plain one gives, and the oracle."""
+    import torch
+    hq, dt = hkv * group, pa_amd.FP8_E4M3 if fp8 else pa_amd.FP16
+    q, k, v, table, ks, vs = paged_inputs(len(lens), lens, hq, hkv, 16, fp8, seed=len(lens))
+    plan = _plan(fp8, lens, group, hkv, 0)
+    dplan = pa_amd.DevicePlan()
+    dplan.upload(plan, group, D)
+    outs = []
+    for static in (False, True):
+        p = pa_amd.DecodeParams()
+        out = torch.full_like(q, float("nan"))
+        p.q, p.k_cache, p.v_cache, p.block_table = q.data_ptr(), k.data_ptr(), v.data_ptr(), table.data_ptr()
+        p.out, p.block_table_stride = out.data_ptr(), table.size(1)
+        p.batch, p.num_q_heads, p.num_kv_heads, p.head_dim, p.page_size = len(lens), hq, hkv, D, 16
+        p.sm_scale, p.k_scale, p.v_scale = pa_amd.sm_scale(D), ks, vs
+        dplan.bind(p)
+        assert p.num_segments == len(plan.segments)
+        if static:
+            pa_amd._lib.call("pa_decode_static", dt, ctypes.byref(p), p.num_segments, None)
+        else:
+            pa_amd.paged_decode(dt, p)
+        torch.cuda.synchronize()
+        outs.append(out)
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+    kb = k.view(torch.uint8).cpu().numpy() if fp8 else k.view(torch.int16).cpu().numpy().view(np.uint16)
+    vb = v.view(torch.uint8).cpu().numpy() if fp8 else v.view(torch.int16).cpu().numpy().view(np.uint16)
+    ref = oracle.paged_decode(dt, q.view(torch.int16).cpu().numpy().view(np.uint16), kb, vb, table.cpu().numpy(),
+                              np.asarray(lens, np.int32), hq, hkv, D, 16, ks, vs, threads=16)
+    assert float(np.max(np.abs(outs[1].float().cpu().numpy() - ref))) < TOL
+
+
+@pytest.mark.parametrize("lens,fp8,group,hkv", [
     ([200], False, 4, 8),                          # one item per block, fewer blocks than the chip has
     ([33], False, 2, 8),                           # three tiles per item
     ([200] * 32, False, 4, 8),                     # as many items as blocks

@@ -94,6 +94,17 @@ def test_decode_static_sizes_no_workspace_for_unsplit_or_block_merged_plans():
     assert st not in (_lib.PA_OK, _lib.PA_ERR_LENGTH) and b"static scratch" not in lib.pa_last_error()
 
 
+def test_decode_static_takes_joined_tiles_without_a_workspace():
+    """block_merge 4 (inside one block, segments joined from single tiles) writes no partial either."""
+    lib = _lib.load()
+    p = pa_amd.DecodeParams()
+    p.num_q_heads, p.num_kv_heads, p.head_dim, p.num_ctas, p.batch = 32, 8, D, 2048, 4
+    p.num_segments, p.needs_merge, p.block_merge = 16384, 0, 4
+    st = lib.pa_decode_static(0, ctypes.byref(p), 16384, None)
+    assert st not in (_lib.PA_OK, _lib.PA_ERR_LENGTH) and b"static scratch" not in lib.pa_last_error()
+    assert b"split rows" not in lib.pa_last_error()
+
+
 @pytest.mark.gpu
 @pytest.mark.usefixtures("gpu_device")
 @pytest.mark.parametrize("fp8", [False, True], ids=["fp16", "fp8"])
