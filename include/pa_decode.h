@@ -144,6 +144,13 @@ int       pa_plan_num_ctas(const pa_plan* plan);
 int       pa_plan_tile(const pa_plan* plan);
 int       pa_plan_num_segments(const pa_plan* plan);
 int       pa_plan_num_items(const pa_plan* plan);
+/* Whether the plan's grid is pa_plan_build's own choice (num_ctas <= 0): only
+ * such a plan's segments may run on other units than its own (see
+ * pa_device_plan_upload). Plans from arrays start as 0; a binding that copied a
+ * plan out (pa_plan_copy) hands the answer on with the setter. No counterpart in
+ * the reference. */
+int       pa_plan_own_grid(const pa_plan* plan);
+pa_status pa_plan_set_own_grid(pa_plan* plan, int own);
 /* How the split kernel merges this plan's split items: 1 or 2 as
  * DevicePlan::bind sets pa_decode_params.block_merge (see there), 0 where the
  * merge kernel finishes them (bind then sets needs_merge, and block_merge 3 if
@@ -167,7 +174,8 @@ void      pa_device_plan_destroy(pa_device_plan* dp);
  * synchronize the stream (it waits only when 8 of its uploads are still in
  * flight, and synchronizes once when a plan outgrows every earlier one), and
  * the host plan may change or go as soon as it returns. Decodes queued earlier
- * on `stream` still see the previous plan. */
+ * on `stream` still see the previous plan. A plan of pa_plan_build's own grid may
+ * run with its segments grouped on other units (bind's num_ctas and block_merge). */
 pa_status pa_device_plan_upload(pa_device_plan* dp, const pa_plan* plan, int group, int head_dim,
                                 void* stream);
 /* decode.cu:148-156 DevicePlan::bind: points the schedule fields of *p at it. */

@@ -24,6 +24,7 @@ struct DecodePlan {
     std::vector<int4> segments;
     std::vector<int>  cta_seg_begin;
     std::vector<int>  item_seg_begin;
+    bool              own_grid = false;   // make_plan chose num_ctas: an upload may group the segments on other units
 };
 
 // Tokens per planning tile for this configuration (the kernel's step).
@@ -62,6 +63,7 @@ inline DecodePlan to_plan(const pa_plan* h) {
     p.item_seg_begin.resize(static_cast<size_t>(pa_plan_num_items(h)) + 1);
     check(pa_plan_copy(h, reinterpret_cast<int32_t*>(p.segments.data()), p.cta_seg_begin.data(),
                        p.item_seg_begin.data()));
+    p.own_grid = pa_plan_own_grid(h) != 0;
     return p;
 }
 }  // namespace detail
@@ -94,6 +96,7 @@ public:
                                      static_cast<int>(plan.segments.size()), plan.cta_seg_begin.data(),
                                      plan.item_seg_begin.data(), items, 0, &raw));
         detail::PlanHandle h(raw);
+        detail::check(pa_plan_set_own_grid(raw, plan.own_grid ? 1 : 0));
         detail::check(pa_device_plan_upload(h_, h.get(), group, head_dim, stream));
     }
     void bind(DecodeParams& p) const { detail::check(pa_device_plan_bind(h_, detail::abi(p))); }

@@ -35,7 +35,8 @@ struct pa_plan {
     std::vector<int32_t> cta_seg_begin;   // [num_ctas + 1]
     std::vector<int32_t> item_seg_begin;  // [items + 1]
     pa_split_shape       shape;
-    int per = 0;   // tiles per unit if the plan is an equal cut as make_plan's, else 0
+    int  per      = 0;       // tiles per unit if the plan is an equal cut as make_plan's, else 0
+    bool own_grid = false;   // nobody asked for its grid: make_plan chose it
 };
 
 // One pinned host staging buffer for host-to-device copies on a stream: pinned

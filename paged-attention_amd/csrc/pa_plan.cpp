@@ -64,6 +64,7 @@ void cut(pa_plan& plan, int tile, const int32_t* lens, int batch, int hkv, int r
     plan.tile     = tile;
     plan.items    = batch * hkv;
     plan.per      = 0;
+    plan.own_grid = false;
 
     long total = 0;
     for (int b = 0; b < batch; ++b) {
@@ -224,8 +225,10 @@ void make_plan_impl(pa_plan& plan, int dtype, const int32_t* lens, int batch, in
     const int group = group_of(hq, hkv);
     check_shape(dtype, hd, group);
     const int tile = pa::kernel_tile_tokens(dtype, group);
-    if (num_ctas <= 0) num_ctas = wave_ctas_impl(dtype, hd, group);
+    const bool own = num_ctas <= 0;
+    if (own) num_ctas = wave_ctas_impl(dtype, hd, group);
     cut(plan, tile, lens, batch, hkv, num_ctas);
+    plan.own_grid = own;
 }
 
 namespace {
@@ -261,12 +264,12 @@ constexpr double kSpanUs16 = 1.2, kSpanUs32 = 2.0;   // fp16, FP8 (16- and 32-to
 // across blocks by the estimate, for longer segments inside would cost precision
 // and uneven units time: fp16 32 x 1000, 32 x 5000, 128 rows of 100 to 200, FP8 32 x
 // 2000 (22.3, 97, 16.4 and 23.0 when segments were cut anew; 24.7, 102, 17.9, 25.5).
-// Only for the plan that make_plan gives a grid of its own choice (`units`), whoever
-// brings it: another grid is the caller's. The host plan stays as it is.
+// Only for a plan whose grid make_plan chose (`units`; own_grid): another grid is the
+// caller's, also where it has as many tiles per unit. The host plan stays as it is.
 // False: not grouped, `out` holds nothing of use.
 bool group_in_blocks(const pa_plan& plan, int units, pa_plan& out) {
     const int items = plan.items, max_blocks = units / pa::kBlockUnits;
-    if (items <= 0 || max_blocks <= 0 || plan.per <= 0) return false;
+    if (!plan.own_grid || items <= 0 || max_blocks <= 0 || plan.per <= 0) return false;
     auto tiles = [&](int sg) {
         const int32_t* s = &plan.segments[4 * static_cast<size_t>(sg)];
         return (s[3] - s[2] + plan.tile - 1) / plan.tile;
@@ -671,6 +674,13 @@ int  pa_plan_num_ctas(const pa_plan* plan) { return plan ? plan->num_ctas : 0; }
 int  pa_plan_tile(const pa_plan* plan) { return plan ? plan->tile : 0; }
 int  pa_plan_num_segments(const pa_plan* plan) { return plan ? static_cast<int>(plan->segments.size() / 4) : 0; }
 int  pa_plan_num_items(const pa_plan* plan) { return plan ? plan->items : 0; }
+int pa_plan_own_grid(const pa_plan* plan) { return plan && plan->own_grid ? 1 : 0; }
+pa_status pa_plan_set_own_grid(pa_plan* plan, int own) {
+    return guarded([&] {
+        if (!plan) throw std::invalid_argument("plan is null");
+        plan->own_grid = own != 0;
+    });
+}
 pa_status pa_plan_merge_mode(const pa_plan* plan, int* out) {
     return guarded([&] {
         if (!plan || !out) throw std::invalid_argument("plan or out is null");

@@ -118,6 +118,8 @@ SIGNATURES: dict[str, tuple] = {
     "pa_plan_tile": (_I, [_P]),
     "pa_plan_num_segments": (_I, [_P]),
     "pa_plan_num_items": (_I, [_P]),
+    "pa_plan_own_grid": (_I, [_P]),
+    "pa_plan_set_own_grid": (_I, [_P, _I]),
     "pa_plan_merge_mode": (_I, [_P, _PI]),
     "pa_plan_copy": (_I, [_P, _P, _P, _P]),
     "pa_device_plan_create": (_I, [_PP]),

@@ -296,6 +296,17 @@ void gpu_checks() {
         "append past max_pages_per_slot");
     HIP_CHECK(hipFree(d));
 
+    // Only a plan whose grid was left to make_plan may run on other units.
+    for (const int asked : {0, 104}) {
+        const decode::DecodePlan plan = decode::make_plan(decode::KVDtype::FP16, {200}, 32, 8, kD, asked);
+        decode::DevicePlan dplan;
+        dplan.upload(plan, 4, kD);
+        decode::DecodeParams dp{};
+        dplan.bind(dp);
+        expect(plan.num_ctas == 104 && plan.own_grid == (asked == 0), "13 tiles x 8 heads, one per unit");
+        expect(asked == 0 ? dp.block_merge == 4 : dp.block_merge == 2 && dp.num_ctas == 104, "an asked-for grid stays");
+    }
+
     // ContiguousKVStore round trip (include/kv_store.hpp).
     std::vector<float> hk(4 * kD, 1.5f), hv(4 * kD, -2.f);
     ContiguousKVStore store(hk.data(), hv.data(), 4, kD);

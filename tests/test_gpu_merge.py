@@ -240,7 +240,8 @@ def test_grouping_keeps_the_partials(lens, fp8, group, hkv):
 def test_another_grid_is_left_as_it_is():
     """A caller's grid, and rows that are cheaper across blocks, keep the host plan's arrays."""
     for lens, ctas in (([200] * 32, 512), ([500], 0), ([300, 1000, 450, 700] * 8, 0),
-                       ([100, 150, 200, 130, 170, 110, 190, 120] * 16, 0)):
+                       ([100, 150, 200, 130, 170, 110, 190, 120] * 16, 0),
+                       ([48], 24), ([200], 104), ([200] * 32, 2048)):   # as many tiles per unit as without a grid
         plan = _plan(False, lens, 4, 8, ctas)
         assert plan.merge_mode == 2
         dplan = pa_amd.DevicePlan()

@@ -77,6 +77,24 @@ def test_product_equals_oracle_and_invariants(seed):
     _check_invariants(plan, lens, hkv, tile, requested)
 
 
+def test_a_plan_knows_whether_its_grid_was_asked_for():
+    """A grid that the caller names is the caller's, also through plans made from arrays; a binding may say otherwise."""
+    import ctypes
+    lib = pa_amd._lib.load()
+    for plan in (pa_amd.make_plan(pa_amd.FP16, [48], 32, 8, 128, 24), pa_amd.make_plan_tiled(16, [48], 8, 24)):
+        assert lib.pa_plan_own_grid(plan.handle.value) == 0
+    segs, cta, item = (np.ascontiguousarray(a) for a in (plan.segments, plan.cta_seg_begin, plan.item_seg_begin))
+    h = ctypes.c_void_p()
+    pa_amd._lib.call("pa_plan_create", plan.num_ctas, 16, segs.ctypes.data, len(segs), cta.ctypes.data,
+                     item.ctypes.data, len(item) - 1, 8, ctypes.byref(h))
+    assert lib.pa_plan_own_grid(h.value) == 0
+    pa_amd._lib.call("pa_plan_set_own_grid", h.value, 1)
+    assert lib.pa_plan_own_grid(h.value) == 1
+    lib.pa_plan_destroy(h.value)
+    assert lib.pa_plan_own_grid(None) == 0
+    assert lib.pa_plan_set_own_grid(None, 1) == pa_amd._lib.PA_ERR_INVALID_ARGUMENT
+
+
 def test_make_plan_uses_kernel_tile_and_validates():
     plan = pa_amd.make_plan(pa_amd.FP16, [8192] * 32, 32, 8, 128, 1024)
     assert plan.tile == pa_amd.tile_tokens(pa_amd.FP16, 128, 4) == 16
