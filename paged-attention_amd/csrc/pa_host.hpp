@@ -12,7 +12,9 @@
 #include <cstdint>
 #include <new>
 #include <stdexcept>
+#include <chrono>
 #include <string>
+#include <thread>
 #include <vector>
 
 // How a plan's split items lie in units and blocks.
@@ -50,6 +52,7 @@ struct pa_stage {
     size_t     cap  = 0;   // int32 elements, marks not counted
     size_t     marks = 0;  // marks of the last copy (at host + cap), one per block
     int32_t    mark  = 0;  // their value once it has read the buffer
+    hipStream_t queue = nullptr;   // where that copy was queued
     bool       captured = false;   // a graph's copy kernel reads it: kept as it is until the pool goes
     hipEvent_t done = nullptr;
 };
@@ -165,7 +168,25 @@ void release_stage(pa_stage& st, hipStream_t s);
 // buffer as read: no event. (An event between two kernels of a stream costs 4 us
 // of the stream's time.)
 void copy_stage(pa_stage& st, int32_t* dev, size_t n, hipStream_t s);
-// Waits for every queued use of the pool and frees its buffers and events.
+// Waits until read() holds, which work on some queue is to bring about, and asks
+// status() about that queue now and then: hipErrorNotReady while it works,
+// hipSuccess once it is through (then one more look decides), else what stopped it.
+template <class Read, class Status>
+hipError_t wait_read(Read&& read, Status&& status) {
+    for (int i = 0; !read(); ++i) {
+        if (i < 4096) {   // a few ms: a copy behind a few decodes has come by then
+            std::this_thread::yield();
+            continue;
+        }
+        const hipError_t e = status();
+        if (e == hipSuccess) return read() ? hipSuccess : hipErrorUnknown;
+        if (e != hipErrorNotReady) return e;
+        std::this_thread::sleep_for(std::chrono::microseconds(20));
+    }
+    return hipSuccess;
+}
+// Waits for every queued use of the pool (not past an error of the device) and
+// frees its buffers and events.
 void free_stages(pa_stage_pool& sp);
 
 // ---- planner and device plan (pa_plan.cpp)

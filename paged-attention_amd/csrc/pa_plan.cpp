@@ -9,7 +9,6 @@
 #include <algorithm>
 #include <climits>
 #include <string>
-#include <thread>
 #include <vector>
 
 namespace {
@@ -375,6 +374,25 @@ bool stage_read(const pa_stage& st) {
         if (__atomic_load_n(st.host + st.cap + i, __ATOMIC_ACQUIRE) != st.mark) return false;
     return true;
 }
+// What the queue of that copy is at (pa::host::wait_read's status).
+hipError_t queue_status(hipStream_t s) {
+    // A query ends the capture of a stream that is being captured.
+    hipStreamCaptureMode   mode = hipStreamCaptureModeRelaxed;
+    hipStreamCaptureStatus cs   = hipStreamCaptureStatusNone;
+    hipError_t e = hipThreadExchangeStreamCaptureMode(&mode);
+    if (e != hipSuccess) return e;
+    e = hipStreamIsCapturing(s, &cs);
+    if (e == hipSuccess) e = cs == hipStreamCaptureStatusNone ? hipStreamQuery(s) : hipErrorNotReady;
+    // The caller's stream may be gone; its work is not.
+    if (e == hipErrorContextIsDestroyed || e == hipErrorInvalidHandle) e = hipDeviceSynchronize();
+    if (e == hipErrorStreamCaptureImplicit || e == hipErrorStreamCaptureUnsupported) e = hipErrorNotReady;
+    if (e == hipErrorNotReady) (void)hipGetLastError();   // an answer, not an error of the next launch
+    const hipError_t back = hipThreadExchangeStreamCaptureMode(&mode);
+    return back == hipSuccess ? e : back;
+}
+hipError_t wait_stage(const pa_stage& st) {
+    return wait_read([&] { return stage_read(st); }, [&] { return queue_status(st.queue); });
+}
 bool stage_idle(const pa_stage& st) {
     if (!stage_read(st)) return false;
     if (!st.done) return true;
@@ -398,7 +416,7 @@ pa_stage& take_stage(pa_stage_pool& sp, size_t need, bool with_device) {
             sp.bufs.emplace_back();
         } else {
             pick = oldest;   // every buffer in flight
-            while (!stage_read(sp.bufs[pick])) std::this_thread::yield();
+            pa::hip_check(wait_stage(sp.bufs[pick]), "staging copy");
             if (sp.bufs[pick].done)
                 pa::hip_check(hipEventSynchronize(sp.bufs[pick].done), "hipEventSynchronize staging");
         }
@@ -441,13 +459,14 @@ void copy_stage(pa_stage& st, int32_t* dev, size_t n, hipStream_t s) {
     }
     st.mark  = st.mark == INT32_MAX ? 1 : st.mark + 1;
     st.marks = pa::stage_copy_blocks(n);
+    st.queue = s;
     const hipError_t e = pa::launch_stage_copy(st.host_dev, dev, n, st.host_dev + st.cap, st.mark, s);
     if (e != hipSuccess) st.marks = 0;   // nothing was queued
     pa::hip_check(e, "staging copy kernel launch");
 }
 void free_stages(pa_stage_pool& sp) {
     for (pa_stage& st : sp.bufs) {
-        while (!stage_read(st)) std::this_thread::yield();
+        (void)wait_stage(st);
         if (st.done) (void)hipEventSynchronize(st.done);
         (void)hipHostFree(st.host);
         (void)hipFree(st.dev);

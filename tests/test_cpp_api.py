@@ -40,3 +40,8 @@ def test_legacy_api_host():
 @pytest.mark.gpu
 def test_legacy_api_device():
     _run("gpu", "test_legacy_api")
+
+
+def test_wait_for_a_staging_copy_ends():
+    """A plan's upload or release waits for its copies, but not for one that a failed queue will never run."""
+    _run("cpu", "test_wait")

@@ -121,3 +121,40 @@ def test_uploads_beyond_the_staging_buffers_and_in_a_graph():
                 decode(lens_of[i], outs[i], side, plans[i])
             torch.cuda.synchronize()
             assert all(torch.equal(alone[i], outs[i]) for i in range(12))
+
+
+def test_uploads_behind_long_work():
+    """More uploads than staging buffers on a stream that is busy for tens of milliseconds: the call waits, asking
+    the stream, and every decode runs under its own plan."""
+    import torch
+    from helpers import paged_inputs
+    lens_of = [[40 * (i + 1), 5, 300 + i] for i in range(12)]
+    q, k, v, table, ks, vs = paged_inputs(3, [600] * 3, 8, 2, 16, False, seed=3)
+    side, dplan = torch.cuda.Stream(), pa_amd.DevicePlan()
+    plans = [pa_amd.make_plan(pa_amd.FP16, lens, 8, 2, D) for lens in lens_of]
+    big = torch.randn((8192, 8192), device="cuda")
+
+    def decode(i, out):
+        dplan.upload(plans[i], 4, D, side)
+        p = pa_amd.DecodeParams()
+        p.q, p.k_cache, p.v_cache, p.block_table = q.data_ptr(), k.data_ptr(), v.data_ptr(), table.data_ptr()
+        p.out, p.block_table_stride = out.data_ptr(), table.size(1)
+        p.batch, p.num_q_heads, p.num_kv_heads, p.head_dim, p.page_size = 3, 8, 2, D, 16
+        p.sm_scale, p.k_scale, p.v_scale = pa_amd.sm_scale(D), ks, vs
+        dplan.bind(p)
+        pa_amd.paged_decode(pa_amd.FP16, p, side)
+
+    alone = [torch.empty_like(q) for _ in lens_of]
+    outs = [torch.empty_like(q) for _ in lens_of]
+    torch.cuda.synchronize()
+    for i, o in enumerate(alone):
+        decode(i, o)
+        torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        for _ in range(6):
+            big = big @ big
+            big = big / big.norm()
+        for i, o in enumerate(outs):
+            decode(i, o)
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, o) for a, o in zip(alone, outs))
