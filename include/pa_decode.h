@@ -339,7 +339,9 @@ pa_status pa_cache_append(pa_cache* cache, int slot, const uint16_t* d_k, const 
  * (copy or E4M3 quantize), no stream synchronization: they travel in its
  * arguments, or, past about 3.5 KB (some 290 new pages), through pinned staging
  * and a copy kernel before it. Then the call waits only when 8 such batches are
- * still in flight. */
+ * still in flight. Captured into a graph, every replay stores the tokens then at
+ * d_k / d_v at the same positions; a slot is released only once the replays that
+ * write to it are done (the cache cannot tell). */
 pa_status pa_cache_append_batch(pa_cache* cache, const int32_t* slots, const int32_t* counts, int n,
                                 const uint16_t* d_k, const uint16_t* d_v, void* stream, int* appended);
 /* paged_kv_cache.cu:138-146 release. The slot's length on the device becomes

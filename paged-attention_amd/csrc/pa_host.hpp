@@ -162,8 +162,10 @@ inline hipStream_t as_stream(void* s) { return static_cast<hipStream_t>(s); }
 // one, else (kMaxStages in flight) the oldest after waiting for it. Grows a
 // buffer by reallocating. The reference is valid until the next take_stage.
 pa_stage& take_stage(pa_stage_pool& sp, size_t need, bool with_device);
-// Records the buffer's event on s: call after queuing the work that reads it.
+// Records the buffer's event on s: call after queuing the work that reads it. On
+// a stream that is being captured the buffer is kept for the graph's replays.
 void release_stage(pa_stage& st, hipStream_t s);
+bool capturing(hipStream_t s);   // whether work queued on s goes into a graph
 // Queues the copy kernel of the buffer's first n ints to dev, which marks the
 // buffer as read: no event. (An event between two kernels of a stream costs 4 us
 // of the stream's time.)

@@ -133,9 +133,10 @@ void queue_append(pa_cache& c, const int32_t* slots, const int32_t* counts, int 
         pa::hip_check(pa::launch_stage_copy(st->host_dev, st->dev, need, nullptr, 0, s), "append staging kernel launch");
     pa::hip_check(pa::launch_append_batch(c.cfg.dtype, a, in_args ? meta : nullptr, need, s), "append kernel launch");
     // Tells a later use of the buffer, and release, when this append is done
-    // (release works on the null stream, which orders itself after its own work).
+    // (release works on the null stream, which orders itself after its own work;
+    // nothing tells of a graph's replays).
     if (!in_args) release_stage(*st, s);
-    else if (s) mark_append(c, s);
+    else if (s && !capturing(s)) mark_append(c, s);
 }
 
 // Notes a stream the cache's work is queued on.
@@ -256,11 +257,11 @@ pa_status pa_cache_append(pa_cache* c, int slot, const uint16_t* d_k, const uint
         if (static_cast<long long>(n) * c->cfg.num_kv_heads * (pa::kHeadDim / 8) > INT_MAX)
             throw std::length_error("append: n * num_kv_heads * 16 exceeds INT_MAX");
         const int old_len = slot_ok(c->pool, slot) ? c->pool.seq_lens[static_cast<size_t>(slot)] : 0;
+        const hipStream_t s = n > 0 ? append_stream(*c, stream) : nullptr;
         int first_new = 0, num_new = 0;
         if (!pool_reserve(c->pool, slot, n, first_new, num_new)) return;   // out of pages: nothing appended
         if (appended) *appended = 1;
         if (n <= 0) return;
-        const hipStream_t s = append_stream(*c, stream);
         const std::vector<reserve_entry> entry{{old_len, first_new, num_new}};
         queue_append(*c, &slot, &n, 1, entry, n, d_k, d_v, s);
         pa::hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
@@ -277,12 +278,12 @@ pa_status pa_cache_append_batch(pa_cache* c, const int32_t* slots, const int32_t
         const int hkv = c->cfg.num_kv_heads;
         if (n_tok * hkv * (pa::kHeadDim / 8) > INT_MAX) throw std::length_error("append_batch: too many tokens");
         if (n_tok > 0 && (!d_k || !d_v)) throw std::invalid_argument("append_batch: k or v is null");
+        const hipStream_t s = n_tok > 0 ? append_stream(*c, stream) : nullptr;
         std::vector<reserve_entry> entries;
         if (!pool_reserve_batch(c->pool, slots, counts, n, &entries)) return;   // out of pages: nothing appended
         if (appended) *appended = 1;
         if (n_tok == 0) return;
-
-        queue_append(*c, slots, counts, n, entries, n_tok, d_k, d_v, append_stream(*c, stream));
+        queue_append(*c, slots, counts, n, entries, n_tok, d_k, d_v, s);
     });
 }
 

@@ -445,14 +445,21 @@ pa_stage& take_stage(pa_stage_pool& sp, size_t need, bool with_device) {
     }
     return st;
 }
+bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (s) pa::hip_check(hipStreamIsCapturing(s, &cs), "hipStreamIsCapturing");
+    return cs != hipStreamCaptureStatusNone;
+}
 void release_stage(pa_stage& st, hipStream_t s) {
+    if (capturing(s)) {
+        st.captured = true;
+        return;
+    }
     if (!st.done) pa::hip_check(hipEventCreateWithFlags(&st.done, hipEventDisableTiming), "hipEventCreate");
     pa::hip_check(hipEventRecord(st.done, s), "hipEventRecord staging");
 }
 void copy_stage(pa_stage& st, int32_t* dev, size_t n, hipStream_t s) {
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (s) pa::hip_check(hipStreamIsCapturing(s, &cs), "hipStreamIsCapturing");
-    if (cs != hipStreamCaptureStatusNone) {   // the graph's replays read it
+    if (capturing(s)) {   // the graph's replays read it
         pa::hip_check(pa::launch_stage_copy(st.host_dev, dev, n, nullptr, 0, s), "staging copy kernel launch");
         st.captured = true;
         return;

@@ -158,3 +158,47 @@ def test_uploads_behind_long_work():
             decode(i, o)
     torch.cuda.synchronize()
     assert all(torch.equal(a, o) for a, o in zip(alone, outs))
+
+
+@pytest.mark.parametrize("n", [7, 400], ids=["in_arguments", "staged"])
+def test_captured_append_after_a_release_on_the_null_stream(n):
+    """A release queued on the null stream, then an append to the same slot captured on another: the wait for the
+    release leaves the capture whole, and every replay stores the tokens then in the inputs, with the page list of
+    its own batch, whatever appends ran in between (400 one-token pages are 1205 ints of metadata: past the kernel's
+    arguments). Releases after it find no event that only a graph has."""
+    import torch
+    hkv, rows = 2, 2000
+    cache = pa_amd.PagedKVCache(rows, 1, hkv, D, 8, 420)
+    x, y = (torch.randn((420, hkv, D), dtype=torch.float16, device="cuda") for _ in range(2))
+    first = cache.admit()
+    assert cache.append_batch([first], [3], x, x, 0)
+    assert cache.append_batch([cache.admit()], [400], x, x, 0)   # staging buffers are made outside captures
+    graph, tokens, side = torch.cuda.CUDAGraph(), x.clone(), torch.cuda.Stream()
+    with torch.cuda.graph(graph, stream=side):
+        cache.release(first)
+        slot = cache.admit()
+        assert slot == first
+        assert cache.append_batch([slot], [n], tokens, tokens, torch.cuda.current_stream())
+    p = cache.params()
+    pages = cache.block_table(slot)
+    assert cache.seq_len(slot) == n and len(pages) == n
+
+    def kept():
+        from helpers import d2h
+        k = d2h(int(p.k_cache), rows * hkv * D * 2, np.uint16).reshape(rows, hkv, D)
+        return k[list(pages)]
+
+    for rep in range(3):
+        tokens.copy_(x if rep % 2 else y)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(kept(), tokens[:n].view(torch.int16).cpu().numpy().view(np.uint16))
+        assert int(d2h(p.seq_lens, 4 * 8, np.int32)[slot]) == n
+        other = cache.admit()          # eager appends of other shapes between the replays
+        assert cache.append_batch([other], [390 + rep], y, y, side)
+        torch.cuda.synchronize()
+        assert int(d2h(p.seq_lens, 4 * 8, np.int32)[other]) == 390 + rep
+        cache.release(other)
+        assert int(d2h(p.seq_lens, 4 * 8, np.int32)[other]) == 0
+    cache.close()
