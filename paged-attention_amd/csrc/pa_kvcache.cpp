@@ -262,8 +262,31 @@ pa_status pa_cache_append(pa_cache* c, int slot, const uint16_t* d_k, const uint
         if (!pool_reserve(c->pool, slot, n, first_new, num_new)) return;   // out of pages: nothing appended
         if (appended) *appended = 1;
         if (n <= 0) return;
-        const std::vector<reserve_entry> entry{{old_len, first_new, num_new}};
-        queue_append(*c, &slot, &n, 1, entry, n, d_k, d_v, s);
+        const int P = c->cfg.page_size, pages = (old_len + n - 1) / P - old_len / P + 1;
+        if (pa::append_meta_inline(3 + static_cast<size_t>(pages) + 2 * (static_cast<size_t>(num_new) + 1))) {
+            const std::vector<reserve_entry> entry{{old_len, first_new, num_new}};
+            queue_append(*c, &slot, &n, 1, entry, n, d_k, d_v, s);
+        } else {
+            // This call waits in any case, so the new table entries go over from
+            // where they are. Through a staging buffer the pages went three times
+            // (list, entries, from there to the kernel): us a call, that way and this,
+            // 131072 tokens of one-token pages 453 / 222, 16384 71 / 49 to 69, 2000
+            // 24 / 25, and the first on a cache, which had the buffer to make, 52 / 27.
+            int32_t* row = c->d_table + static_cast<size_t>(slot) * c->cfg.max_pages_per_slot;
+            const auto& table = c->pool.tables[static_cast<size_t>(slot)];
+            pa::hip_check(hipMemcpyAsync(row + first_new, table.data() + first_new,
+                                         sizeof(int32_t) * static_cast<size_t>(num_new), hipMemcpyHostToDevice, s),
+                          "hipMemcpyAsync block table");
+            pa::hip_check(hipMemcpyAsync(c->d_seq_lens + slot, &c->pool.seq_lens[static_cast<size_t>(slot)],
+                                         sizeof(int32_t), hipMemcpyHostToDevice, s),
+                          "hipMemcpyAsync seq_len");
+            const bool  fp8   = c->cfg.dtype == PA_KV_FP8_E4M3;
+            const float inv_k = fp8 ? 1.0f / c->cfg.k_scale : 1.0f;
+            const float inv_v = fp8 ? 1.0f / c->cfg.v_scale : 1.0f;
+            pa::hip_check(pa::launch_append(c->cfg.dtype, d_k, d_v, c->d_k, c->d_v, row, old_len, n,
+                                            c->cfg.num_kv_heads, P, inv_k, inv_v, s),
+                          "append kernel launch");
+        }
         pa::hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
     });
 }

@@ -1,6 +1,7 @@
 """Appends whose page lists sit at the edges of what travels in a kernel's arguments (256 and 896 ints; past
-that through a staging buffer), one call per sequence and batched, and on more streams than are tracked:
-stored bytes bit-exact, decode within tolerance, device table and lengths as the host's.
+that a batch goes through a staging buffer, a single append by copies), one call per sequence and batched,
+and on more streams than are tracked: stored bytes bit-exact, decode within tolerance, device table and
+lengths as the host's.
 """
 
 from __future__ import annotations
