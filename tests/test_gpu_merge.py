@@ -237,6 +237,43 @@ def test_grouping_keeps_the_partials(lens, fp8, group, hkv):
     assert float((apart > 0).float().mean()) < 2.0 ** -3
 
 
+@pytest.mark.parametrize("factors", [[60.0, 0.1], [0.1, 60.0], [60.0, 30.0, 1.0, 0.0], [0.0]], ids=str)
+def test_joined_tiles_far_apart(factors):
+    """Tiles of one segment whose largest scores lie hundreds of powers of two apart, in either order, and tiles of
+    equal scores: each is scored against its own maximum or, far below, counts nothing; finite, and as across blocks."""
+    import torch
+    lens, group, hkv, hq = [200], 4, 8, 32
+    q, k, v, table, ks, vs = paged_inputs(1, lens, hq, hkv, 16, False, seed=23)
+    for j, page in enumerate(table[0].tolist()[:13]):
+        k[page] *= factors[j % len(factors)]
+    plan = _plan(False, lens, group, hkv, 0)
+    asked = _plan(False, lens, group, hkv, plan.num_ctas)   # the same cut, on its own units
+    outs = []
+    for pl, mode in ((plan, 4), (asked, 2)):
+        dplan = pa_amd.DevicePlan()
+        dplan.upload(pl, group, D)
+        p = pa_amd.DecodeParams()
+        out = torch.full_like(q, float("nan"))
+        p.q, p.k_cache, p.v_cache, p.block_table = q.data_ptr(), k.data_ptr(), v.data_ptr(), table.data_ptr()
+        p.out, p.block_table_stride = out.data_ptr(), table.size(1)
+        p.batch, p.num_q_heads, p.num_kv_heads, p.head_dim, p.page_size = 1, hq, hkv, D, 16
+        p.sm_scale, p.k_scale, p.v_scale = pa_amd.sm_scale(D), ks, vs
+        dplan.bind(p)
+        assert p.block_merge == mode
+        pa_amd.paged_decode(pa_amd.FP16, p)
+        torch.cuda.synchronize()
+        outs.append(out.float())
+    assert torch.isfinite(outs[0]).all()
+    # Two fp16 roundings of fp32 averages of the same partials, of values below 4.5.
+    assert float((outs[0] - outs[1]).abs().max()) <= 2.0 ** -8
+    kb, vb = (x.view(torch.int16).cpu().numpy().view(np.uint16) for x in (k, v))
+    ref = oracle.paged_decode(pa_amd.FP16, q.view(torch.int16).cpu().numpy().view(np.uint16), kb, vb,
+                              table.cpu().numpy(), np.asarray(lens, np.int32), hq, hkv, D, 16, ks, vs, threads=16)
+    # Scores of several hundred carry the rounding of their fp32 sums (2^-24 of sums below 2^13: 2^-11 in the
+    # exponent, so 2^-11 of a weight) besides what the ordinary cases have.
+    assert float(np.max(np.abs(outs[0].cpu().numpy() - ref))) < TOL + 4.5 * 2.0 ** -11
+
+
 def test_another_grid_is_left_as_it_is():
     """A caller's grid, and rows that are cheaper across blocks, keep the host plan's arrays."""
     for lens, ctas in (([200] * 32, 512), ([500], 0), ([300, 1000, 450, 700] * 8, 0),
