@@ -186,8 +186,9 @@ __global__ __launch_bounds__(256) void append_kernel(const uint16_t* __restrict_
 }
 
 // An append whose meta travels in the kernel's arguments (N ints): no staging
-// buffer, no copy before the kernel. A decode step's tokens of up to 128
-// sequences fit, and prompts of some 290 new pages.
+// buffer, no copy before the kernel. A decode step's tokens of 112 sequences fit
+// where each begins a page, of up to 149 where none does (6 ints a sequence and
+// 2 a new page), and prompts of some 290 new pages.
 template <int N>
 struct AppendInline {
     AppendBatch a;

@@ -25,6 +25,32 @@ def test_meta_sizes(fp8, batched, lens):
     assert err <= TOL
 
 
+@pytest.mark.parametrize("n,prefix", [(112, 0), (113, 0), (149, 1), (150, 1), (128, 3)], ids=str)
+def test_decode_step_meta_sizes(n, prefix):
+    """One token to each of n sequences: 8 n ints of metadata where each begins a page (896 and 904), 6 n where none
+    does (894 and 900); the last with every sequence at the end of a page, so that 128 new entries go along (1024)."""
+    import torch
+    P, hkv = (1, 2) if prefix == 0 else (3 if prefix == 3 else 4, 2)
+    cache = pa_amd.PagedKVCache(2 * n + 5, P, hkv, D, n, 4)
+    cache.shuffle_free_pages(3)
+    slots = [cache.admit() for _ in range(n)]
+    x = torch.randn((n * max(prefix, 1), hkv, D), dtype=torch.float16, device="cuda")
+    y = torch.randn((n, hkv, D), dtype=torch.float16, device="cuda")
+    if prefix:
+        assert cache.append_batch(slots, [prefix] * n, x, x, 0)
+    assert cache.append_batch(slots, [1] * n, y, x, 0)
+    p = cache.params()
+    assert list(d2h(int(p.seq_lens), 4 * n, np.int32)) == [prefix + 1] * n
+    table = d2h(int(p.block_table), 16 * n, np.int32).reshape(n, 4)
+    k = d2h(int(p.k_cache), (2 * n + 5) * hkv * P * D * 2, np.uint16).reshape(-1, hkv, P, D)
+    want = y.view(torch.int16).cpu().numpy().view(np.uint16)
+    for i, s in enumerate(slots):
+        pages = cache.block_table(s)
+        assert list(table[s, :len(pages)]) == list(pages) and len(pages) == prefix // P + 1
+        assert np.array_equal(k[pages[prefix // P], :, prefix % P], want[i])
+    cache.close()
+
+
 def test_appends_on_many_streams_then_release():
     """Ten streams append to a sequence each (more than the cache tracks at once); device lengths and tables are
     the host's, and a released slot's length is zero on the device."""
