@@ -410,7 +410,7 @@ def workload_figures(s, desc: str, steps: int, warmup: int, cold_iters: int, flu
     nbytes = s.bytes()
     step_us = wall * 1e6 / steps
     split_us = (region_ms / steps if s.params.needs_merge == 0 else statistics.mean(split_ms)) * 1e3
-    out = {"workload": desc, "page_size": s.page, "units": s.plan.num_ctas, "segments": int(len(s.plan.segments)),
+    out = {"workload": desc, "page_size": s.page, "units": int(s.params.num_ctas), "segments": int(len(s.plan.segments)),
            "merge": merge_of(s), "algorithmic_bytes": nbytes,
            "us_per_step": round(step_us, 2), "pct_of_peak": round(100 * nbytes / (step_us * 1e-6) / 1e9 / PEAK_GBPS, 2),
            "split_us": round(split_us, 2),
@@ -477,7 +477,7 @@ def main() -> None:
     desc, _, _, _, fp8 = CONFIGS[args.config]
     print(f"# bench: {desc}, page_size {args.page_size}", file=sys.stderr, flush=True)
     s = bd.Setup(seq_lens_of(args.config), HQ, HKV, D, args.page_size, fp8, shuffle=True, ctas=args.ctas)
-    print(f"# setup done: {s.batch} seqs, {s.num_pages} pages, plan {s.plan.num_ctas} units / "
+    print(f"# setup done: {s.batch} seqs, {s.num_pages} pages, {int(s.params.num_ctas)} units / "
           f"{len(s.plan.segments)} segments", file=sys.stderr, flush=True)
 
     nbytes = s.bytes()
@@ -540,7 +540,7 @@ def main() -> None:
             "head_dim": D,
             "page_size": args.page_size,
             "kv_dtype": "fp8_e4m3" if fp8 else "fp16",
-            "units": s.plan.num_ctas,
+            "units": int(s.params.num_ctas),   # as they run; segments as planned
             "segments": int(len(s.plan.segments)),
             "merge": merge_of(s),
             "algorithmic_bytes": nbytes,

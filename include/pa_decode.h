@@ -151,11 +151,11 @@ int       pa_plan_num_items(const pa_plan* plan);
  * the reference. */
 int       pa_plan_own_grid(const pa_plan* plan);
 pa_status pa_plan_set_own_grid(pa_plan* plan, int own);
-/* How the split kernel merges this plan's split items: 1 or 2 as
- * DevicePlan::bind sets pa_decode_params.block_merge (see there), 0 where the
- * merge kernel finishes them (bind then sets needs_merge, and block_merge 3 if
- * the blocks merge their own parts first). No counterpart in
- * the reference, whose plans always merge in a second kernel
+/* How the split kernel merges this plan's split items on the plan's own units:
+ * 1 inside one block, 2 across blocks, 0 where the merge kernel finishes them.
+ * What a device plan runs as, bind says (pa_decode_params.block_merge): for 0
+ * with needs_merge, 3 if the blocks merge their own parts first; for a 2 whose
+ * upload groups the segments inside blocks, 1 or 4. No counterpart in the reference, whose plans always merge in a second kernel
  * (decode.cu:143 needs_merge). Pure host. */
 pa_status pa_plan_merge_mode(const pa_plan* plan, int* out);
 /* Copies segments ([n][4]), cta_seg_begin ([num_ctas+1]) and item_seg_begin

@@ -99,12 +99,13 @@ hipError_t launch_append_batch(int dtype, const AppendBatch& a, const int32_t* m
 // Whether an append's meta of n ints fits the kernel arguments (4 KiB in all).
 constexpr size_t kAppendInlineInts = 896;
 constexpr bool   append_meta_inline(size_t n) { return n <= kAppendInlineInts; }
-// Stores one zero. Copies n ints (rounded up to whole 16 bytes) from pinned host memory to the
+// Stores one zero.
+hipError_t launch_zero_int(int32_t* p, hipStream_t s);
+// Copies n ints (rounded up to whole 16 bytes) from pinned host memory to the
 // device with a kernel. Both ends are 16-byte aligned and have that room. Block i
 // of stage_copy_blocks(n) stores `mark` at marks[i] (pinned host memory; null:
 // none) once it has read its part.
 constexpr size_t stage_copy_blocks(size_t n) { return (n + 1023) / 1024; }
-hipError_t launch_zero_int(int32_t* p, hipStream_t s);
 hipError_t launch_stage_copy(const int32_t* host, int32_t* dev, size_t n, int32_t* marks, int32_t mark, hipStream_t s);
 hipError_t launch_gather(int dtype, const void* cache, const int32_t* bt_row, int hkv,
                          int page_size, int kv_head, int len, void* out, hipStream_t s);

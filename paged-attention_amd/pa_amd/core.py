@@ -132,9 +132,10 @@ class DecodePlan:
 
     @property
     def merge_mode(self) -> int:
-        """How the plan's split items are merged: 0 (merge kernel; bind may have
-        the blocks merge their own parts first), 1 (split items merged inside
-        one block), 2 (items spanning blocks merged by the split kernel too)."""
+        """How the plan's split items are merged on its own units: 0 (merge kernel), 1
+        (inside one block), 2 (across blocks, by the split kernel). A device plan may
+        run otherwise: bind's block_merge is 3 where the blocks merge their own parts
+        for the merge kernel, 1 or 4 where an upload groups a 2 inside blocks."""
         if self.handle is None:
             raise ValueError("plan has no native handle")
         out = ctypes.c_int(0)
