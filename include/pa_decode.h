@@ -175,7 +175,9 @@ void      pa_device_plan_destroy(pa_device_plan* dp);
  * flight, and synchronizes once when a plan outgrows every earlier one), and
  * the host plan may change or go as soon as it returns. Decodes queued earlier
  * on `stream` still see the previous plan. A plan of pa_plan_build's own grid may
- * run with its segments grouped on other units (bind's num_ctas and block_merge). */
+ * run with its segments grouped on other units (bind's num_ctas and block_merge).
+ * An upload captured into a graph keeps its staging buffer, for the replays, until
+ * the device plan is destroyed. */
 pa_status pa_device_plan_upload(pa_device_plan* dp, const pa_plan* plan, int group, int head_dim,
                                 void* stream);
 /* decode.cu:148-156 DevicePlan::bind: points the schedule fields of *p at it. */
@@ -341,7 +343,7 @@ pa_status pa_cache_append(pa_cache* cache, int slot, const uint16_t* d_k, const 
  * and a copy kernel before it. Then the call waits only when 8 such batches are
  * still in flight. Captured into a graph, every replay stores the tokens then at
  * d_k / d_v at the same positions; a slot is released only once the replays that
- * write to it are done (the cache cannot tell). */
+ * write to it are done (the cache cannot tell), and staging goes with the cache. */
 pa_status pa_cache_append_batch(pa_cache* cache, const int32_t* slots, const int32_t* counts, int n,
                                 const uint16_t* d_k, const uint16_t* d_v, void* stream, int* appended);
 /* paged_kv_cache.cu:138-146 release. The slot's length on the device becomes
